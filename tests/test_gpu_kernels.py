@@ -327,6 +327,40 @@ def test_the_tiled_gemm_at_the_prefill_shapes(kernels, name, rows, cols):
     assert (p.view(np.uint32) == f.view(np.uint32)).all(), f"{name}: panels"
 
 
+@pytest.mark.parametrize("rows,cols,n", [(64, 4096, 65), (1000, 2056, 65), (260, 12288, 100), (516, 4104, 200),
+                                         (4096, 4096, 257), (1024, 3072, 777), (2052, 1032, 333), (4, 1024, 65)])
+def test_the_gemm_of_few_tiles_cuts_k_into_slices(kernels, rows, cols, n):
+    """Gpu::gemm past 64 rows where the tiles are too few for the chip: the K slices and their
+    reduction, at ends inside a tile, a stage and a slice. Against float64 products within the
+    GEMV tolerance for f32 sums, the bf16 output the f32 output rounded, the same bits on a
+    second call, from panels where W's rows are a multiple of 16, and replayed from a graph."""
+    rng = np.random.default_rng(rows + cols + n)
+    w = O.bf16_round(rng.normal(0, 0.02, rows * cols).astype(np.float32))
+    x = O.bf16_round(rng.normal(0, 1.0, n * cols).astype(np.float32))
+    f = kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, True)
+    W, X = w.reshape(rows, cols).astype(np.float64), x.reshape(n, cols).astype(np.float64)
+    r = np.abs(f.astype(np.float64) - X @ W.T) / (1e-5 * (np.abs(X) @ np.abs(W).T) + 1e-30)
+    assert (r <= 1.0).all(), f"worst ratio {r.max():.3f}"
+    b = kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, False)
+    assert (b == bf16_bits(f).reshape(b.shape)).all()
+    assert (kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, True).view(np.uint32) == f.view(np.uint32)).all()
+    if rows % 16 == 0:
+        p = kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, True, tile=0, layout=W_PANELS | X_PANELS)
+        assert (p.view(np.uint32) == f.view(np.uint32)).all()
+    from x0ne_core import Arena, Class
+    g, a = kernels.gpu, Arena()
+    ws, xs, ys = (a.alloc(k, v, Class.CLIENT_DATA) for k, v in (("w", w.size * 2), ("x", x.size * 2), ("y", n * rows * 4)))
+    a.freeze(g)
+    a.write(ws, 0, bf16_bits(w))
+    a.write(xs, 0, bf16_bits(x))
+    graph = g.capture(lambda: g.gemv(a.ptr(ws), rows, cols, a.ptr(xs), n, a.ptr(ys), True))
+    for _ in range(3):
+        a.write(ys, 0, np.zeros(n * rows, np.float32))
+        g.launch_graph(graph)
+        g.sync()
+        assert (a.read_array(ys, 0, n * rows, np.uint32) == f.view(np.uint32).ravel()).all()
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_few_row_gemm_is_the_oracle_and_its_swiglu_the_swiglu_kernel(kernels, seed):
     """The batched step's projection kernel (2 to 64 rows of X, each W row read once) at every

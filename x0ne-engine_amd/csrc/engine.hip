@@ -434,7 +434,7 @@ struct x0ne_engine {
     // A prefill pass's rows: f32 residual, bf16 delta, normed x, qkv, q, attention, [gate; up], act.
     x0ne_slice p_res{}, p_delta{}, p_x{}, p_qkv{}, p_q{}, p_attn{}, p_gu{}, p_act{};
     x0ne_slice p_tok{};  // a batched engine's pass of several sequences: their ids side by side
-    x0ne_slice p_parts{};  // the exact mode's prefill GEMM: f64 partial sums of K slices
+    x0ne_slice p_parts{};  // a pass's GEMMs: the K slices' partial sums (f64 in the exact mode, else f32)
     // The batched step's rows ([max_batch][...]): f32 residual, bf16 delta, normed x, qkv,
     // attention, SwiGLU activation, f32 logits; its split-K state and counters.
     x0ne_slice b_res{}, b_delta{}, b_x{}, b_qkv{}, b_attn{}, b_act{}, b_logits{}, b_state{}, b_counter{}, b_argmax{};
@@ -507,6 +507,20 @@ struct x0ne_greedy {
 };
 
 namespace {
+
+// The room for the K slices of a pass of up to `chunk` rows: the most that a layer's projections
+// take, looked at every 8 rows (a count between that would take more gets fewer slices).
+uint64_t tile_parts_bytes(const x0ne_engine* e) {
+    const Cfg& c = e->c;
+    const uint64_t shapes[4][2] = {{c.qkv_rows(), c.hidden}, {c.hidden, c.q_dim()}, {2 * c.inter, c.hidden}, {c.hidden, c.inter}};
+    uint64_t most = 0;
+    for (const auto& s : shapes)
+        for (uint64_t n = 65; n <= e->chunk; n += 8) {
+            const uint32_t k = x0ne_gemm_tile_plan((uint32_t)s[0], (uint32_t)s[1], (uint32_t)n, e->gpu->cus, TILE_PARTS_BYTES).slices;
+            if (k > 1) most = std::max(most, k * n * s[0] * 4);
+        }
+    return most;
+}
 
 x0ne_status plan(x0ne_engine* e) {
     x0ne_arena* a = e->arena;
@@ -601,6 +615,10 @@ x0ne_status plan(x0ne_engine* e) {
         X0NE_TRY(al("prefill_act", np * c.inter * 2, CD, &e->p_act));
         if (e->max_batch > 1) X0NE_TRY(al("prefill_ids", n * 4, CD, &e->p_tok));
         if (e->f64_sums) X0NE_TRY(al("prefill_f64_parts", EXACT_PARTS_BYTES, CD, &e->p_parts));
+        // One sequence's f32 passes cut the K of their few-tile GEMMs into slices. A batched engine
+        // keeps every sum in one piece: a sequence's bits must not depend on the rows beside it.
+        if (const uint64_t bytes = e->f64_sums || e->max_batch > 1 ? 0 : tile_parts_bytes(e))
+            X0NE_TRY(al("prefill_f32_parts", bytes, CD, &e->p_parts));
     }
     if (e->max_batch > 1) {
         const uint64_t b = e->max_batch, bp = (b + 15) / 16 * 16;  // panels hold whole tiles of 16 rows
@@ -950,12 +968,13 @@ x0ne_status gemm(x0ne_engine* e, x0ne_slice w, x0ne_slice w_panels, uint64_t row
     if (e->f64_sums)
         return exact_gemm(e->gpu, e->d(w), rows, cols, e->d(x), n, e->d(y), false, (double*)e->d(e->p_parts),
                           EXACT_PARTS_BYTES);
+    const TileWork work = e->p_parts.len ? TileWork{(float*)e->d(e->p_parts), e->p_parts.len} : TileWork{};
     if (!e->ppanel)
-        return x0ne_gpu_gemv(e->gpu, (uint64_t)(uintptr_t)e->d(w), rows, cols, (uint64_t)(uintptr_t)e->d(x), n,
-                             (uint64_t)(uintptr_t)e->d(y), 0);
+        return gemv_rows(e->gpu, (uint64_t)(uintptr_t)e->d(w), rows, cols, (uint64_t)(uintptr_t)e->d(x), n,
+                         (uint64_t)(uintptr_t)e->d(y), false, work);
     if (n <= 64) return skinny(e->gpu, e->d(w_panels), rows, cols, e->d(x), n, e->d(y), 0, PANEL_X | PANEL_W);
     return tiled_gemm(e->gpu, 0, X0NE_GEMM_W_PANELS | X0NE_GEMM_X_PANELS, e->d(w_panels), rows, cols, e->d(x), n,
-                      e->d(y), false);
+                      e->d(y), false, work);
 }
 
 // Prompt rows pos0 .. pos0 + n - 1 through every layer (engine.rs:729-839 with n rows): the
@@ -1195,7 +1214,7 @@ x0ne_status capture(x0ne_engine* e) {
         x0ne_graph_free(e->graph);
         e->graph = nullptr;
     }
-    X0NE_TRY(x0ne_gpu_capture_begin(e->gpu));
+    X0NE_TRY(capture_begin(e->gpu));
     x0ne_status st = step_launches(e);
     x0ne_graph* gr = nullptr;
     x0ne_status st2 = x0ne_gpu_capture_end(e->gpu, &gr);
@@ -2045,7 +2064,7 @@ x0ne_status batch_capture(x0ne_engine* e, uint32_t B) {
         e->bgraph = nullptr;
         e->bgraph_batch = 0;
     }
-    X0NE_TRY(x0ne_gpu_capture_begin(e->gpu));
+    X0NE_TRY(capture_begin(e->gpu));
     x0ne_status st = batch_step_launches(e, B);
     x0ne_graph* gr = nullptr;
     x0ne_status st2 = x0ne_gpu_capture_end(e->gpu, &gr);

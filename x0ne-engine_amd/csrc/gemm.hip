@@ -637,12 +637,16 @@ extern "C" __global__ void __launch_bounds__(256)
 //    (rotating weights).
 //  - A load past the matrix (a token past n, a feature past rows, k past cols) is a buffer load
 //    at an offset past the buffer: zeros, no memory touched.
-//  - Tiles in launch order go round the 8 XCDs (each with its own L2): the launch's blocks are
-//    renumbered so each XCD takes a contiguous run of tiles, and runs are ordered TILE_GROUP
-//    feature tiles wide, tokens fastest, so the blocks an XCD holds at once share their W and X
-//    pieces in its L2.
-// Each output is summed over k by one wavefront in a fixed order: bit-reproducible, and the
-// same bits whatever the operands' layout.
+//  - A launch of few tiles cuts K into `slices` equal runs of stages (x0ne_gemm_tile_plan): block
+//    (slice, tile) writes its f32 sums to parts[slice][token][feature] and
+//    x0ne_gemm_tiles_reduce adds the slices in slice order. 200 x 4096 x 12288: 64 tiles, 158 us;
+//    32 tiles of 256 x 128 in 8 slices, 40 us with the reduction (floor 16 us, W at 6.5 TB/s).
+//  - Blocks in launch order go round the 8 XCDs (each with its own L2): they are renumbered so
+//    each XCD takes a contiguous run of (slice, tile), tiles fastest, and a slice's tiles are
+//    ordered TILE_GROUP feature tiles wide, tokens slowest, so the blocks an XCD holds at once
+//    share their W and X pieces in its L2 (with 8 slices, each XCD reads its own eighth of K).
+// Each output is summed over k by one wavefront per slice in a fixed order: bit-reproducible, and
+// with one slice the same bits whatever the tile, the operands' layout or the number of tokens.
 namespace {
 
 constexpr int TILE_GROUP = 4;  // feature tiles side by side in one run of tiles
@@ -700,14 +704,15 @@ constexpr int WAIT_LGKM0 = 0xC07F;
 template <int WF, int WT, int NWF, int NWT, int STAGES>
 __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const bf16_t* __restrict__ x,
                                            void* __restrict__ y, uint32_t rows, uint32_t cols, uint32_t n,
-                                           uint32_t flags, uint8_t* lds) {
+                                           uint32_t flags, uint32_t slices, float* __restrict__ parts, uint8_t* lds) {
     using C = TileCfg<WF, WT, NWF, NWT, STAGES>;
     const uint32_t tiles_f = (rows + C::BF - 1) / C::BF, tiles_t = (n + C::BT - 1) / C::BT;
-    const uint32_t tiles = tiles_f * tiles_t;
-    // Launch id -> tile: ids alternate over the 8 XCDs, so id b runs on XCD b % 8; the XCD's
-    // ids b % 8, b % 8 + 8, .. take the run of tiles (b % 8) (tiles / 8) + b / 8.
-    const uint32_t b = blockIdx.x;
-    const uint32_t seq = tiles % 8 == 0 ? (b & 7) * (tiles >> 3) + (b >> 3) : b;
+    const uint32_t tiles = tiles_f * tiles_t, total = tiles * slices;
+    // Launch id -> (slice, tile): ids alternate over the 8 XCDs, so block b runs on XCD b % 8; the
+    // XCD's blocks b % 8, b % 8 + 8, .. take a contiguous run of total / 8 (and one of the rest).
+    const uint32_t b = blockIdx.x, xcd = b & 7;
+    const uint32_t id = xcd * (total >> 3) + min(xcd, total & 7) + (b >> 3);
+    const uint32_t slice = id / tiles, seq = id - slice * tiles;
     const uint32_t group = seq / (TILE_GROUP * tiles_t), in_group = seq % (TILE_GROUP * tiles_t);
     const uint32_t width = min((uint32_t)TILE_GROUP, tiles_f - group * TILE_GROUP);
     const uint32_t f0 = (group * TILE_GROUP + in_group % width) * C::BF, t0 = in_group / width * C::BT;
@@ -718,7 +723,10 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
     // Panels hold whole groups of 16 rows.
     const i32x4 wr = rsrc_words(w, (uint64_t)(w_panel ? (rows + 15) / 16 * 16 : rows) * cols * 2);
     const i32x4 xr = rsrc_words(x, (uint64_t)(x_panel ? (n + 15) / 16 * 16 : n) * cols * 2);
-    const uint32_t stages = (cols + 32 * TILE_K - 1) / (32 * TILE_K), c8 = cols / 8;
+    const uint32_t all = (cols + 32 * TILE_K - 1) / (32 * TILE_K), c8 = cols / 8;
+    // This slice's stages: first, first + 1, .. (counted from 0 below).
+    const uint32_t first = (uint32_t)((uint64_t)all * slice / slices);
+    const uint32_t stages = (uint32_t)((uint64_t)all * (slice + 1) / slices) - first;
 
     // This wavefront's loads of a stage: load h (0, 1) of 16-row group g = wave + NW (q / 2) (W's
     // groups first). In panels lane l fetches row l % 16, columns 32 h + 8 (l / 16) .. + 7 of the
@@ -737,7 +745,8 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
         row_in[q] = row < (is_w ? rows : n);
         step[q] = TILE_K * (panel ? 1024 : 64);
         chunk0[q] = panel ? 4 * h + (lane >> 4) : (lane & 7) ^ (lane >> 3);
-        base[q] = panel ? g16 * c8 * 256 + 1024 * h + 16 * lane : row * cols * 2 + 16 * chunk0[q];
+        base[q] = (panel ? g16 * c8 * 256 + 1024 * h + 16 * lane : row * cols * 2 + 16 * chunk0[q]) + step[q] * first;
+        chunk0[q] += 4 * TILE_K * first;
     }
     auto issue = [&](uint32_t s) {
         uint8_t* dst = lds + (s % STAGES) * C::BYTES;
@@ -854,7 +863,9 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
             if (f >= rows) continue;
             const f32x4 v = acc[i][j];
             const size_t o = (size_t)t * rows + f;
-            if (out_f32) {
+            if (slices > 1) {
+                *reinterpret_cast<f32x4*>(parts + (size_t)slice * n * rows + o) = v;
+            } else if (out_f32) {
                 *reinterpret_cast<f32x4*>(static_cast<float*>(y) + o) = v;
             } else {
                 const uint32_t lo = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
@@ -867,26 +878,53 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
 
 }  // namespace
 
-// Tiled GEMM kernels: grid ceil(rows / BF) ceil(n / BT), block 64 NWF NWT; rows a multiple of 4,
-// cols of 8 (and rows of 16 with W in panels), W and X below 4 GiB - 16 bytes, Y 8-byte (bf16)
-// or 16-byte (f32) aligned; flags TILE_F32 | TILE_W_PANEL | TILE_X_PANEL.
+// Tiled GEMM kernels: grid ceil(rows / BF) ceil(n / BT) slices, block 64 NWF NWT; rows a multiple
+// of 4, cols of 8 (and rows of 16 with W in panels), W and X below 4 GiB - 16 bytes, Y 8-byte
+// (bf16) or 16-byte (f32) aligned; flags TILE_F32 | TILE_W_PANEL | TILE_X_PANEL; slices at most
+// the stages of K, parts [slices][n][rows] f32 when more than one.
 #define X0NE_TILES(NAME, WF, WT, NWF, NWT, STAGES)                                                              \
     extern "C" __global__ void __launch_bounds__(64 * NWF * NWT)                                                      \
         NAME(const bf16_t* __restrict__ w, const bf16_t* __restrict__ x, void* __restrict__ y, uint32_t rows,         \
-             uint32_t cols, uint32_t n, uint32_t flags) {                                                             \
+             uint32_t cols, uint32_t n, uint32_t flags, uint32_t slices, float* __restrict__ parts) {                 \
         __shared__ __attribute__((aligned(1024))) uint8_t lds[STAGES * TileCfg<WF, WT, NWF, NWT, STAGES>::BYTES];     \
-        if (rows % 4 != 0 || cols % 8 != 0 || n == 0 || ((flags & TILE_W_PANEL) && rows % 16 != 0)) return;         \
-        gemm_tiles<WF, WT, NWF, NWT, STAGES>(w, x, y, rows, cols, n, flags, lds);                                     \
+        if (rows % 4 != 0 || cols % 8 != 0 || n == 0 || slices == 0 || ((flags & TILE_W_PANEL) && rows % 16 != 0))    \
+            return;                                                                                                   \
+        gemm_tiles<WF, WT, NWF, NWT, STAGES>(w, x, y, rows, cols, n, flags, slices, parts, lds);                      \
     }
-// Block tiles from sweeps on MI355X over the Qwen3 prefill shapes, as many stages as fit the LDS:
-// 256 x 256 of 8 wavefronts (64 features x 128 tokens each; two per SIMD; four stages of 32
-// columns in their place: 5-7 % slower row-major, level in panels), 256 x 128 of 8 (64 x 64 each)
-// and 128 x 128 of 4 (64 x 64 each).
+// Block tiles from sweeps on MI355X over the Qwen3 projections at 65 to 2048 rows of X: 256 x 256
+// of 8 wavefronts (64 features x 128 tokens each; two per SIMD; four stages of 32 columns in
+// their place: 5-7 % slower row-major, level in panels), 256 x 128 of 8 (64 x 64 each), 64 x 64 of 4
+// (32 x 32 each, two blocks per CU), and 128 x 128 of 4, which a caller may name but no shape
+// is best on.
 X0NE_TILES(x0ne_gemm_tiles_256x256_bf16, 64, 128, 4, 2, 2)
 X0NE_TILES(x0ne_gemm_tiles_256x128_bf16, 64, 64, 4, 2, 3)
 X0NE_TILES(x0ne_gemm_tiles_128x128_bf16, 64, 64, 2, 2, 4)
+X0NE_TILES(x0ne_gemm_tiles_64x64_bf16, 32, 32, 2, 2, 4)
+
+// x0ne_gemm_tiles_reduce: y[t][f] = the f32 (flags TILE_F32) or bf16 of the sum over slices, in
+// slice order, of parts[slice][t][f]; one thread per 4 features, grid ceil(n rows / 4 / 256),
+// block 256; rows a multiple of 4. Bound by the parts' reads (from the L2 and the Infinity Cache).
+extern "C" __global__ void __launch_bounds__(256)
+    x0ne_gemm_tiles_reduce(const float* __restrict__ parts, void* __restrict__ y, uint32_t rows, uint32_t n,
+                           uint32_t flags, uint32_t slices) {
+    const uint64_t quads = (uint64_t)n * rows / 4, i = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    if (rows % 4 != 0 || i >= quads) return;
+    const f32x4* p = reinterpret_cast<const f32x4*>(parts) + i;
+    f32x4 v = p[0];
+    for (uint32_t s = 1; s < slices; ++s) v += p[s * quads];
+    if (flags & TILE_F32) {
+        static_cast<f32x4*>(y)[i] = v;
+    } else {
+        const uint32_t lo = (uint32_t)f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16);
+        const uint32_t hi = (uint32_t)f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16);
+        static_cast<uint2*>(y)[i] = make_uint2(lo, hi);
+    }
+}
 
 // ---- typed launchers of the tiled GEMM (called by the runtime) ----
+
+#include <algorithm>
+#include <cmath>
 
 #include "launch.h"
 
@@ -894,39 +932,75 @@ namespace {
 
 struct TileKind {
     const void* fn;
-    uint32_t bf, bt;    // block tile: features x tokens
+    uint32_t bf, bt;  // block tile: features x tokens
     uint32_t threads;
+    // The plan's estimate, us on MI355X: a block's start and end, and one stage with a block on
+    // every CU (64 x 64: with one block on the CU; two or more take `shared` each).
+    double fixed, stage, shared;
 };
 
 TileKind tile_kind(int tile) {
     switch (tile) {
-        case X0NE_TILE_256x256: return {(const void*)&x0ne_gemm_tiles_256x256_bf16, 256, 256, 512};
-        case X0NE_TILE_256x128: return {(const void*)&x0ne_gemm_tiles_256x128_bf16, 256, 128, 512};
-        case X0NE_TILE_128x128: return {(const void*)&x0ne_gemm_tiles_128x128_bf16, 128, 128, 256};
-        default: return {nullptr, 0, 0, 0};
+        case X0NE_TILE_256x256: return {(const void*)&x0ne_gemm_tiles_256x256_bf16, 256, 256, 512, 6.8, 1.45, 1.45};
+        case X0NE_TILE_256x128: return {(const void*)&x0ne_gemm_tiles_256x128_bf16, 256, 128, 512, 5.7, 0.95, 0.95};
+        case X0NE_TILE_128x128: return {(const void*)&x0ne_gemm_tiles_128x128_bf16, 128, 128, 256, 0, 0, 0};
+        case X0NE_TILE_64x64: return {(const void*)&x0ne_gemm_tiles_64x64_bf16, 64, 64, 256, 3.6, 0.27, 0.235};
+        default: return {nullptr, 0, 0, 0, 0, 0, 0};
     }
+}
+
+uint64_t tile_count(const TileKind& k, uint32_t rows, uint32_t n) {
+    return (uint64_t)((rows + k.bf - 1) / k.bf) * ((n + k.bt - 1) / k.bt);
 }
 
 }  // namespace
 
-// The tile for a shape, from the MI355X sweeps at 2048 rows of X (operands in panels): the
-// 256 x 256 tile while it gives at least 0.7 of a tile per CU (gate/up 24576 rows: 335-360 us;
-// QKV 6144 rows: 98-106 us against 125 for 256 x 128), else 256 x 128 while that does (O and down,
-// 4096 rows: 68 and 186 us against 99 and 278 for 256 x 256), else 128 x 128.
-int x0ne_gemm_tile_pick(uint32_t rows, uint32_t cols, uint32_t n, uint32_t cus) {
-    auto tiles = [&](uint32_t bf, uint32_t bt) { return (uint64_t)((rows + bf - 1) / bf) * ((n + bt - 1) / bt); };
-    if (10 * tiles(256, 256) >= 7ull * cus) return X0NE_TILE_256x256;
-    if (10 * tiles(256, 128) >= 7ull * cus) return X0NE_TILE_256x128;
-    return X0NE_TILE_128x128;
+// The tile and the K slices for a shape: the pair that an estimate of the time puts first. The
+// estimate is a block's fixed and per-stage time times the rounds of blocks over the CUs, not
+// less than W's stream (5.1 TB/s and 2 us), and for several slices the reduction (2.7 us and
+// the parts at 3.7 TB/s). The constants are fitted to a sweep on MI355X of the 12 Qwen3-0.6B,
+// -8B and -32B projections at 17 counts from 65 to 2048 rows, row-major and in panels, weights
+// rotating: over its 396 shapes the picked pair takes 1.7 % longer than the best of 9 tiles x 8
+// slice counts on average, 20 % at worst (777 x 4096 x 12288: 256 x 256 in 4 slices, 92 us;
+// unsplit 256 x 128 159, 256 x 256 251).
+X0neTilePlan x0ne_gemm_tile_plan(uint32_t rows, uint32_t cols, uint32_t n, uint32_t cus, uint64_t parts_bytes) {
+    const uint32_t stages = (cols + 63) / 64;
+    X0neTilePlan best = {X0NE_TILE_256x256, 1};
+    double best_us = 1e30;
+    for (int tile : {X0NE_TILE_64x64, X0NE_TILE_256x128, X0NE_TILE_256x256}) {
+        const TileKind k = tile_kind(tile);
+        for (uint32_t slices : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u}) {
+            const uint64_t part = (uint64_t)n * rows * 4;
+            // A slice holds at least 4 stages, and all slices' blocks come to a few rounds at most.
+            if (slices > 1 && (slices > stages / 4 || slices * part > parts_bytes ||
+                               tile_count(k, rows, n) * slices > 4ull * cus + 64))
+                break;
+            const double per_cu = std::ceil((double)(tile_count(k, rows, n) * slices) / cus);
+            const double steps = std::ceil((double)stages / slices);
+            double us = tile == X0NE_TILE_64x64 ? k.fixed + steps * (per_cu > 1 ? per_cu * k.shared : k.stage)
+                                                : per_cu * (k.fixed + steps * k.stage);
+            const double stream = 2.0 + 2.0 * rows * cols / 5.1e6;
+            us = std::sqrt(std::sqrt(us * us * us * us + stream * stream * stream * stream));
+            if (slices > 1) us += 2.7 + (double)slices * part / 3.7e6;
+            if (us < best_us) best_us = us, best = {tile, slices};
+        }
+    }
+    return best;
 }
 
-hipError_t x0ne_launch_gemm_tiles(int tile, const void* w, const void* x, void* y, uint32_t rows, uint32_t cols,
-                                  uint32_t n, uint32_t flags, hipStream_t s) {
-    const TileKind k = tile_kind(tile);
-    if (!k.fn || rows % 4 != 0 || cols % 8 != 0 || n == 0 || flags > 7 || ((flags & TILE_W_PANEL) && rows % 16 != 0))
+hipError_t x0ne_launch_gemm_tiles(X0neTilePlan plan, const void* w, const void* x, void* y, uint32_t rows, uint32_t cols,
+                                  uint32_t n, uint32_t flags, float* parts, hipStream_t s) {
+    const TileKind k = tile_kind(plan.tile);
+    uint32_t slices = plan.slices;
+    if (!k.fn || rows % 4 != 0 || cols % 8 != 0 || n == 0 || flags > 7 || ((flags & TILE_W_PANEL) && rows % 16 != 0) ||
+        slices == 0 || (slices > 1 && (!parts || slices > (cols + 63) / 64)))
         return hipErrorInvalidValue;
-    const uint64_t blocks = (uint64_t)((rows + k.bf - 1) / k.bf) * ((n + k.bt - 1) / k.bt);
+    const uint64_t blocks = tile_count(k, rows, n) * slices;
     if (blocks > 0x7FFFFFFFull) return hipErrorInvalidValue;
-    void* args[] = {(void*)&w, (void*)&x, (void*)&y, (void*)&rows, (void*)&cols, (void*)&n, (void*)&flags};
-    return x0ne_launch(k.fn, dim3((uint32_t)blocks), dim3(k.threads), args, 0, s);
+    void* args[] = {(void*)&w, (void*)&x, (void*)&y, (void*)&rows, (void*)&cols, (void*)&n, (void*)&flags, (void*)&slices, (void*)&parts};
+    const hipError_t e = x0ne_launch(k.fn, dim3((uint32_t)blocks), dim3(k.threads), args, 0, s);
+    if (e != hipSuccess || slices == 1) return e;
+    void* rargs[] = {(void*)&parts, (void*)&y, (void*)&rows, (void*)&n, (void*)&flags, (void*)&slices};
+    return x0ne_launch((const void*)&x0ne_gemm_tiles_reduce, dim3((uint32_t)(((uint64_t)n * rows / 4 + 255) / 256)),
+                       dim3(256), rargs, 0, s);
 }

@@ -52,6 +52,10 @@ struct x0ne_gpu {
     // This device's copy of the library's static scratch array (runtime.hip, `scratch`), as
     // hipGetSymbolAddress gave it at x0ne_gpu_new with the device current.
     void* scratch = nullptr;
+    // K-slice sums of the tiled GEMM for calls on this Gpu (runtime.hip, tile_work), taken when
+    // first needed and freed with the Gpu. Its calls run on one stream, one after the other.
+    float* tile_parts = nullptr;
+    bool tile_parts_refused = false;  // the allocation failed once: its calls stay unsplit
 };
 
 struct x0ne_graph {
@@ -99,8 +103,21 @@ x0ne_status skinny(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols, con
                    uint32_t mode, uint32_t panels, const FewWork* work = nullptr);
 // The tiled matrix-core GEMM (gemm.hip) behind x0ne_gpu_gemm_tiled: tile 0 picks per shape;
 // layout X0NE_GEMM_W_PANELS | X0NE_GEMM_X_PANELS names the operands held in 16-row panels.
+// With tile 0 a shape of few tiles cuts K into slices when `work` has room for their sums (the
+// same shape and room: the same kernels, the same bits); launches sharing it must not overlap.
+// Without, an output's bits do not depend on n.
+struct TileWork {
+    float* parts = nullptr;
+    uint64_t bytes = 0;
+};
+constexpr uint64_t TILE_PARTS_BYTES = 64ull << 20;  // room for every split that the plan prefers
 x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, uint64_t rows, uint64_t cols,
-                       const void* x, uint64_t n, void* y, bool out_f32);
+                       const void* x, uint64_t n, void* y, bool out_f32, TileWork work = {});
+// x0ne_gpu_gemv with the tiled GEMM's workspace given.
+x0ne_status gemv_rows(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n, uint64_t y,
+                      bool out_f32, TileWork work);
+// x0ne_gpu_capture_begin for a capture that brings its own workspaces.
+x0ne_status capture_begin(x0ne_gpu* g);
 // Y[n][rows] = X[n][cols] W^T with every product summed in f64 (the exact mode's prefill
 // passes; x0ne_gemm_f64_t*_bf16), Y = bf16(f32(sum)) or f32(sum); W and X row-major. ks K slices
 // (0: picked per shape, up to what ws_bytes of ws holds) summed in slice order by

@@ -112,6 +112,7 @@ extern "C" void x0ne_gpu_free(x0ne_gpu* g) {
         (void)hipStreamSynchronize(g->stream);
         (void)hipStreamDestroy(g->stream);
     }
+    if (g->tile_parts) (void)hipFree(g->tile_parts);
     delete g;
 }
 
@@ -282,11 +283,12 @@ namespace x0ne {
 
 // ---- many rows: the tiled matrix-core GEMM of gemm.hip ----
 // The reference hands Gpu::gemm to cuBLAS (gpu.rs:1098-1149); from SKINNY_MAX_ROWS + 1 rows on
-// this library runs its own tiled GEMM (x0ne_launch_gemm_tiles), the tile chosen per shape by
-// x0ne_gemm_tile_pick unless `tile` names one. A shape always runs the same kernel, and each
-// output is summed in a fixed order: results are the same from call to call.
+// this library runs its own tiled GEMM (x0ne_launch_gemm_tiles), the tile and the K slices chosen
+// per shape by x0ne_gemm_tile_plan unless `tile` names one (then unsplit). A shape always runs the
+// same kernels, and each output is summed in a fixed order: results are the same from call to
+// call.
 x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, uint64_t rows, uint64_t cols,
-                       const void* x, uint64_t n, void* y, bool out_f32) {
+                       const void* x, uint64_t n, void* y, bool out_f32, TileWork work) {
     const bool wp = layout & X0NE_GEMM_W_PANELS, xp = layout & X0NE_GEMM_X_PANELS;
     const uint64_t xrows = xp ? (n + 15) / 16 * 16 : n;
     if (rows == 0 || cols == 0 || n == 0 || rows % 4 != 0 || cols % 8 != 0 || (wp && rows % 16 != 0) ||
@@ -296,13 +298,30 @@ x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, ui
         return fail(X0NE_ERR_FORMAT, "tiled gemm: " + std::to_string(rows) + "x" + std::to_string(cols) + ", n " +
                                          std::to_string(n) + " (rows a multiple of 4, of 16 with W in panels, "
                                          "cols of 8, W and X below 4 GiB, 16-byte aligned operands)");
-    if (tile == 0) tile = x0ne_gemm_tile_pick((uint32_t)rows, (uint32_t)cols, (uint32_t)n, g->cus);
+    X0neTilePlan plan = {tile, 1};
+    if (tile == 0)
+        plan = x0ne_gemm_tile_plan((uint32_t)rows, (uint32_t)cols, (uint32_t)n, g->cus, work.parts ? work.bytes : 0);
     const uint32_t flags = (out_f32 ? X0NE_TILE_F32 : 0u) | (wp ? X0NE_TILE_W_PANEL : 0u) | (xp ? X0NE_TILE_X_PANEL : 0u);
     g->counts.gemms++;
-    g->counts.launches++;
-    X0NE_HIP(x0ne_launch_gemm_tiles(tile, w, x, y, (uint32_t)rows, (uint32_t)cols, (uint32_t)n, flags, g->stream),
+    g->counts.launches += plan.slices > 1 ? 2 : 1;
+    X0NE_HIP(x0ne_launch_gemm_tiles(plan, w, x, y, (uint32_t)rows, (uint32_t)cols, (uint32_t)n, flags, work.parts,
+                                    g->stream),
              "tiled gemm");
     return X0NE_OK;
+}
+
+// The Gpu's own workspace for the tiled GEMM's slices, allocated at the first call that may use it
+// or when a capture begins (a capture must not allocate). Without the memory for it the Gpu's
+// GEMMs stay unsplit.
+static TileWork tile_work(x0ne_gpu* g) {
+    if (!g->tile_parts && !g->tile_parts_refused && !g->capturing) {
+        if (hipMalloc((void**)&g->tile_parts, TILE_PARTS_BYTES) != hipSuccess) {
+            (void)hipGetLastError();
+            g->tile_parts = nullptr;
+            g->tile_parts_refused = true;
+        }
+    }
+    return g->tile_parts ? TileWork{g->tile_parts, TILE_PARTS_BYTES} : TileWork{};
 }
 
 x0ne_status skinny(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols, const void* x, uint64_t n, void* y,
@@ -531,12 +550,18 @@ extern "C" x0ne_status x0ne_gpu_gemm_tiled(x0ne_gpu* g, uint32_t tile, uint32_t 
                                            uint64_t cols, uint64_t x, uint64_t n, uint64_t y, int out_f32) {
     if (!g) return fail(X0NE_ERR_GPU, "no device");
     if (tile > X0NE_GEMM_TILE_128x128) return fail(X0NE_ERR_FORMAT, "tiled gemm: tile " + std::to_string(tile));
-    return x0ne::tiled_gemm(g, (int)tile, layout, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32 != 0);
+    return x0ne::tiled_gemm(g, (int)tile, layout, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32 != 0,
+                            tile == X0NE_GEMM_TILE_AUTO ? tile_work(g) : TileWork{});
 }
 
 extern "C" x0ne_status x0ne_gpu_gemv(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n,
                                      uint64_t y, int out_f32) {
     if (!g) return fail(X0NE_ERR_GPU, "no device");
+    return x0ne::gemv_rows(g, w, rows, cols, x, n, y, out_f32 != 0, n > SKINNY_MAX_ROWS ? tile_work(g) : TileWork{});
+}
+
+x0ne_status x0ne::gemv_rows(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n, uint64_t y,
+                            bool out_f32, TileWork work) {
     if (rows == 0 || cols == 0 || n == 0 || rows > UINT32_MAX || cols > UINT32_MAX)
         return fail(X0NE_ERR_FORMAT, "gemv: " + std::to_string(rows) + "x" + std::to_string(cols) + ", n " +
                                          std::to_string(n));
@@ -549,7 +574,7 @@ extern "C" x0ne_status x0ne_gpu_gemv(x0ne_gpu* g, uint64_t w, uint64_t rows, uin
     if (n > SKINNY_MAX_ROWS && cols % 8 == 0 && rows % 4 == 0 && n <= UINT32_MAX &&
         rows * cols * 2 <= GEMM_MAX_BYTES && n * cols * 2 <= GEMM_MAX_BYTES && w % 16 == 0 && x % 16 == 0 &&
         y % 16 == 0)
-        return x0ne::tiled_gemm(g, 0, 0, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32 != 0);
+        return x0ne::tiled_gemm(g, 0, 0, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32, work);
     for (uint64_t r = 0; r < n; ++r) {
         const uint16_t* wp = (const uint16_t*)w;
         const uint16_t* xp = (const uint16_t*)(x + r * cols * 2);
@@ -845,6 +870,12 @@ extern "C" uint64_t x0ne_split_state_bytes(uint32_t q_heads, uint32_t splits) {
 
 extern "C" x0ne_status x0ne_gpu_capture_begin(x0ne_gpu* g) {
     if (!g) return fail(X0NE_ERR_GPU, "no device");
+    if (g->capturing) return fail(X0NE_ERR_GPU, "a capture is already open");
+    (void)tile_work(g);
+    return x0ne::capture_begin(g);
+}
+
+x0ne_status x0ne::capture_begin(x0ne_gpu* g) {
     if (g->capturing) return fail(X0NE_ERR_GPU, "a capture is already open");
     X0NE_HIP(hipStreamBeginCapture(g->stream, hipStreamCaptureModeGlobal), "hipStreamBeginCapture");
     g->capturing = true;
