@@ -505,6 +505,41 @@ def test_the_f64_gemm_is_the_exact_sum_of_the_products(kernels, seed):
     assert equal >= 0.999 * n * rows, f"{what}: {equal} of {n * rows} equal"
 
 
+@pytest.mark.parametrize("kernel,feats,toks", [("t1f1", 16, 16), ("t2f2", 32, 32), ("t3f3", 48, 48)])
+@pytest.mark.parametrize("n,rows,cols,ks", [(1, 1, 8, 1), (49, 65, 264, 1), (33, 33, 1032, 3), (97, 200, 72, 16)])
+def test_the_f64_gemm_at_its_other_tiles(kernels, kernel, feats, toks, n, rows, cols, ks):
+    """The f64-sum GEMM's tiles besides those above, at ends inside a tile, a step and a slice (more
+    slices than steps too): each output the exact sum of its products (math.fsum) rounded to f32,
+    within the f64 sums' own rounding (cols x 2^-53 of the magnitudes, then the f32 rounding)."""
+    import math
+
+    from x0ne_core import Arena, Arg, Class
+    rng = O.Rng(4000 + n + rows)
+    w, x = bf16s_with_edges(rng, rows * cols, 1e-2), bf16s_with_edges(rng, n * cols, 1.0)
+    a, sl = Arena(), {}
+    for name, size in (("w", w.size * 2), ("x", x.size * 2), ("y", n * rows * 4), ("parts", ks * n * rows * 8)):
+        sl[name] = a.alloc(name, size, Class.CLIENT_DATA)
+    a.freeze(kernels.gpu)
+    a.write(sl["w"], 0, bf16_bits(w))
+    a.write(sl["x"], 0, bf16_bits(x))
+    p = {k: Arg.ptr(a.ptr(v)) for k, v in sl.items()}
+    tiles = -(-rows // feats) * -(-n // toks)
+    kernels.gpu.launch(f"x0ne_gemm_f64_{kernel}_bf16", -(-tiles * ks // 4), 256,
+                       [p["w"], p["x"], p["y"], Arg.u32(rows), Arg.u32(cols), Arg.u32(n), Arg.u32(1), Arg.u32(ks), p["parts"]])
+    if ks > 1:
+        kernels.gpu.launch("x0ne_gemm_f64_reduce", -(-n * rows // 256), 256,
+                           [p["parts"], p["y"], Arg.u32(rows), Arg.u32(n), Arg.u32(ks), Arg.u32(1)])
+    kernels.gpu.sync()
+    f = a.read_array(sl["y"], 0, n * rows, np.float32).reshape(n, rows)
+    W, X = w.astype(np.float64).reshape(rows, cols), x.astype(np.float64).reshape(n, cols)
+    for t in range(n):
+        for r in range(rows):
+            terms = X[t] * W[r]
+            exact = math.fsum(terms)
+            bound = cols * 2.0 ** -53 * float(np.abs(terms).sum())
+            assert abs(float(f[t, r]) - exact) <= bound + 0.5 * float(np.spacing(np.float32(abs(exact) + bound))), (t, r)
+
+
 @pytest.mark.parametrize("rows,cols", [(16, 8), (48, 40), (32, 1000), (1024, 4096), (17, 8), (16, 12)])
 def test_panel_copy_is_the_panel_layout(kernels, rows, cols):
     """x0ne_panel_bf16 (the load-time copy of a batched engine's weights) writes the host's panel

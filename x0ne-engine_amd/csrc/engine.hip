@@ -46,7 +46,7 @@ namespace {
 constexpr uint64_t PREFILL_CHUNK = 2048;
 // The exact mode's prefill GEMM: f64 parts of up to this many bytes (a short pass cuts K into
 // slices to fill the chip).
-constexpr uint64_t EXACT_PARTS_BYTES = 32ull << 20;
+constexpr uint64_t EXACT_PARTS_BYTES = 64ull << 20;
 constexpr uint64_t MAX_BATCH = 64;  // the few-row GEMM's most rows
 constexpr uint32_t ARGMAX_SLICES = 64;  // blocks per logits row of the batched step's argmax
 constexpr uint64_t MOE_MAX_EXPERTS = 1024;  // kernels/src/lib.rs:147 (moe.hip)

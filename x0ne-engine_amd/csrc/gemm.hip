@@ -362,7 +362,9 @@ extern "C" __global__ void __launch_bounds__(512)
 //    product's own 4 columns): the same bits from call to call, within f64 rounding of the
 //    oracle's sequential sum.
 //  - A wavefront's steps run one after the other (8 x 16 products of 64 cycles per step at
-//    64 x 64 outputs), so a launch of few tiles (a short prompt) is latency-bound: with ks > 1
+//    64 x 64 outputs), so a launch is as long as the fullest SIMD's wavefronts: 333 x 24576 x 4096
+//    in 64 x 64 tiles is 2.25 wavefronts per SIMD and takes the time of 3. The host picks the
+//    tile (16 x 16, 32 x 32, 48 x 48 or 64 x 32) and the slices of K (exact_gemm); with ks > 1
 //    the steps are cut into ks equal runs, wavefront (tile, slice) writes its f64 partial sums
 //    to ws[slice][token][feature], and x0ne_gemm_f64_reduce adds the slices in slice order.
 // Wavefronts are numbered tokens fastest, then slices, so neighbouring wavefronts share W rows.
@@ -424,15 +426,17 @@ __device__ __forceinline__ void gemm_f64(const bf16_t* __restrict__ w, const bf1
                 for (int t = 0; t < TT; ++t) acc[f][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[f], bv[t], acc[f][t], 0, 0, 0);
         }
     };
-    // Steps in pairs, so each register set is named statically.
+    // Steps in pairs, so each register set is named statically, and no way out between the two: with
+    // one the compiler keeps a second copy of the accumulators and moves them over every pair.
     load(0, s_lo);
-    for (uint32_t s = s_lo; s < steps; s += 2) {
+    uint32_t s = s_lo;
+    for (; s + 1 < steps; s += 2) {
         load(1, s + 1);
         step(0);
-        if (s + 1 >= steps) break;  // wavefront-uniform
         load(0, s + 2);
         step(1);
     }
+    if (s < steps) step(0);
     // acc[f][t][i]: feature 16 (TF ft + f) + l / 16 + 4 i, token 16 (TT tt + t) + l % 16 (the
     // f64 product's result rows interleave over the lane groups).
 #pragma unroll
@@ -460,19 +464,22 @@ __device__ __forceinline__ void gemm_f64(const bf16_t* __restrict__ w, const bf1
 
 }  // namespace
 
-// x0ne_gemm_f64_t{TT}_bf16: grid ceil(ceil(rows / 64) ceil(n / (16 TT)) ks / V), block 64 V
-// threads (any V); cols a multiple of 8; W and X below 4 GiB - 16 bytes; out_f32 0 (bf16 Y) or
-// 1 (f32 Y); ks 1 (Y written) or more (the partial sums into ws: [ks][n][rows] f64, then
-// x0ne_gemm_f64_reduce).
-#define X0NE_GEMM_F64(NAME, TT)                                                                                   \
+// x0ne_gemm_f64_t{TT}[f{TF}]_bf16 (TF 4 unless named): grid ceil(ceil(rows / (16 TF))
+// ceil(n / (16 TT)) ks / V), block 64 V threads (any V); cols a multiple of 8; W and X below
+// 4 GiB - 16 bytes; out_f32 0 (bf16 Y) or 1 (f32 Y); ks 1 (Y written) or more (the partial sums
+// into ws: [ks][n][rows] f64, then x0ne_gemm_f64_reduce).
+#define X0NE_GEMM_F64(NAME, TF, TT)                                                                               \
     extern "C" __global__ void __launch_bounds__(256)                                                              \
         NAME(const bf16_t* __restrict__ w, const bf16_t* __restrict__ x, void* __restrict__ y, uint32_t rows,      \
              uint32_t cols, uint32_t n, uint32_t out_f32, uint32_t ks, double* __restrict__ ws) {                 \
-        gemm_f64<4, TT>(w, x, y, rows, cols, n, out_f32, ks, ws);                                                  \
+        gemm_f64<TF, TT>(w, x, y, rows, cols, n, out_f32, ks, ws);                                                 \
     }
-X0NE_GEMM_F64(x0ne_gemm_f64_t1_bf16, 1)
-X0NE_GEMM_F64(x0ne_gemm_f64_t2_bf16, 2)
-X0NE_GEMM_F64(x0ne_gemm_f64_t4_bf16, 4)
+X0NE_GEMM_F64(x0ne_gemm_f64_t1_bf16, 4, 1)
+X0NE_GEMM_F64(x0ne_gemm_f64_t2_bf16, 4, 2)
+X0NE_GEMM_F64(x0ne_gemm_f64_t4_bf16, 4, 4)
+X0NE_GEMM_F64(x0ne_gemm_f64_t1f1_bf16, 1, 1)
+X0NE_GEMM_F64(x0ne_gemm_f64_t2f2_bf16, 2, 2)
+X0NE_GEMM_F64(x0ne_gemm_f64_t3f3_bf16, 3, 3)
 
 // ---- exact sums for a few rows: 4-token quads ----
 // The same product for n <= 32 rows of X on v_mfma_f64_4x4x4f64, which computes 4 blocks b of
@@ -539,13 +546,14 @@ __device__ __forceinline__ void gemm_f64_quads(const bf16_t* __restrict__ w, con
         }
     };
     load(0, s_lo);
-    for (uint32_t s = s_lo; s < steps; s += 2) {
+    uint32_t s = s_lo;
+    for (; s + 1 < steps; s += 2) {
         load(1, s + 1);
         step(0);
-        if (s + 1 >= steps) break;  // wavefront-uniform
         load(0, s + 2);
         step(1);
     }
+    if (s < steps) step(0);
 #pragma unroll
     for (int f = 0; f < TF; ++f)
 #pragma unroll

@@ -123,7 +123,6 @@ x0ne_status capture_begin(x0ne_gpu* g);
 // (0: picked per shape, up to what ws_bytes of ws holds) summed in slice order by
 // x0ne_gemm_f64_reduce. Launches sharing ws must not overlap.
 constexpr uint32_t EXACT_GEMM_MAX_SLICES = 16;
-constexpr uint32_t EXACT_GEMM_WAVES_PER_CU = 8;
 x0ne_status exact_gemm(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols, const void* x, uint64_t n, void* y,
                        bool out_f32, double* ws, uint64_t ws_bytes, uint32_t ks = 0);
 // Split plan for a geometry (gpu.rs:958-985), P capped at `cap`.

@@ -129,6 +129,9 @@ X0NE_DECLARE_FEW(t4_r1_swiglu)
 X0NE_DECLARE_GEMM_F64(t1)
 X0NE_DECLARE_GEMM_F64(t2)
 X0NE_DECLARE_GEMM_F64(t4)
+X0NE_DECLARE_GEMM_F64(t1f1)
+X0NE_DECLARE_GEMM_F64(t2f2)
+X0NE_DECLARE_GEMM_F64(t3f3)
 X0NE_DECLARE_GEMM_F64(q1)
 X0NE_DECLARE_GEMM_F64(q2)
 X0NE_DECLARE_GEMM_F64(q3)

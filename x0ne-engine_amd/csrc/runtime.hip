@@ -2,6 +2,7 @@
 // x0ne-core/runtime/src/{gpu,arena,error}.rs, on the HIP runtime for gfx950.
 
 #include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -413,6 +414,60 @@ x0ne_status skinny(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols, con
     return X0NE_OK;
 }
 
+// The kernels of the f64-sum GEMM: wavefront tiles of 16 `feats` features by 16 `toks` tokens, and
+// the 4-token quads, which take n <= 32 rows of X in one token tile without padding to 16.
+struct ExactKind {
+    const void* fn;
+    uint32_t feats, toks, quads;  // quads 0: not a quad kernel
+};
+static const ExactKind EXACT_KINDS[] = {
+    {(const void*)&x0ne_gemm_f64_t1f1_bf16, 1, 1, 0}, {(const void*)&x0ne_gemm_f64_t2f2_bf16, 2, 2, 0},
+    {(const void*)&x0ne_gemm_f64_t3f3_bf16, 3, 3, 0}, {(const void*)&x0ne_gemm_f64_t2_bf16, 4, 2, 0},
+    {(const void*)&x0ne_gemm_f64_q1_bf16, 4, 0, 1},   {(const void*)&x0ne_gemm_f64_q2_bf16, 4, 0, 2},
+    {(const void*)&x0ne_gemm_f64_q3_bf16, 4, 0, 3},   {(const void*)&x0ne_gemm_f64_q4_bf16, 4, 0, 4},
+    {(const void*)&x0ne_gemm_f64_q5_bf16, 4, 0, 5},   {(const void*)&x0ne_gemm_f64_q6_bf16, 4, 0, 6},
+    {(const void*)&x0ne_gemm_f64_q7_bf16, 4, 0, 7},   {(const void*)&x0ne_gemm_f64_q8_bf16, 4, 0, 8}};
+struct ExactPlan {
+    const ExactKind* kind = nullptr;
+    uint32_t slices = 1;
+    uint64_t tiles = 0;
+};
+
+// The wavefront tile and the K slices (ks 0: any) that an estimate of the time, us on MI355X, puts
+// first: the wavefronts on the fullest SIMD, 0.25 us per 32-column step and 16 x 16 outputs (a
+// quad's 16 x 4: a quarter, times 1.24), not less than a step's loads (0.09 us and 0.034 per
+// operand piece), W's stream (6.3 TB/s) or the operands' reads from the L2 (8.7 TB/s), then the
+// reduction of the slices (1.1 us and 3.1 TB/s). Fitted to a sweep of the Qwen3-0.6B and -8B
+// projections at 4 to 2048 rows (106 shapes, 21 tiles x 11 slice counts): the picked pair takes
+// 1.03 of the best one's time on average, 1.24 at worst (4 rows); 64 x 64 tiles (quads up to 32
+// rows) in slices to 8 wavefronts per CU, the rule before, 1.58 and 3.5. 333 x 24576 x 4096:
+// 1654 -> 1080 us (1045 at the f64 rate of a large product); 20 x 1024 x 2048: 20 -> 9.3.
+static ExactPlan exact_plan(uint64_t rows, uint64_t cols, uint64_t n, uint32_t cus, uint32_t ks, uint64_t ws_bytes) {
+    ExactPlan best;
+    double best_us = 1e30;
+    const uint64_t steps = (cols + 31) / 32;
+    for (const ExactKind& k : EXACT_KINDS) {
+        if (k.quads && (n > 32 || k.quads != (n + 3) / 4)) continue;
+        const uint64_t tiles = (rows + 16 * k.feats - 1) / (16 * k.feats) * (k.quads ? 1 : (n + 16 * k.toks - 1) / (16 * k.toks));
+        const double outs = k.quads ? 0.25 * k.quads * 1.24 : (double)k.toks;  // in 16 x 16 products
+        const double pieces = k.feats + (k.quads ? k.quads : k.toks);  // 1 KiB operand pieces per step
+        for (uint32_t s : {1u, 2u, 3u, 4u, 5u, 6u, 8u, 12u, 16u}) {
+            if (ks && s != 1) break;
+            const uint32_t slices = ks ? ks : s;
+            if (slices > 1 && !ks && (steps / slices < 4 || slices * n * rows * 8 > ws_bytes)) break;
+            const uint64_t blocks = (tiles * slices + 3) / 4;  // a block's 4 wavefronts: one per SIMD
+            const double work = (double)((blocks + cus - 1) / cus) * k.feats * outs * 0.25;
+            const double loads = 0.09 + 0.034 * pieces;
+            const double stream = 2.0 + 2.0 * rows * cols / 6.3e6, reads = (double)(tiles * steps) * pieces * 1024 / 8.7e6;
+            double us = 2.0 + (double)((steps + slices - 1) / slices) * std::cbrt(work * work * work + loads * loads * loads);
+            us = std::sqrt(std::sqrt(us * us * us * us + stream * stream * stream * stream + reads * reads * reads * reads));
+            if (slices > 1) us += 1.1 + (double)slices * n * rows * 8 / 3.1e6;
+            if (us < best_us) best_us = us, best = {&k, slices, tiles};
+        }
+    }
+    return best;
+}
+
 x0ne_status exact_gemm(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols, const void* x, uint64_t n, void* y,
                        bool out_f32, double* ws, uint64_t ws_bytes, uint32_t ks) {
     if (rows == 0 || cols == 0 || n == 0 || cols % 8 != 0 || rows > UINT32_MAX || n > UINT32_MAX ||
@@ -421,27 +476,9 @@ x0ne_status exact_gemm(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols,
         (ks > 1 && ws == nullptr))
         return fail(X0NE_ERR_FORMAT, "exact gemm: " + std::to_string(rows) + "x" + std::to_string(cols) + ", n " +
                                          std::to_string(n) + ", " + std::to_string(ks) + " slices");
-    // Tokens per wavefront: up to 32 rows of X in quads of 4 (x0ne_gemm_f64_q*, no padding to 16),
-    // beyond that 64 (x0ne_gemm_f64_t4); 64 features per wavefront either way.
-    const uint32_t tq = n <= 32 ? (uint32_t)(n + 3) / 4 : 0, tt = 4;
-    const uint64_t tiles = (rows + 63) / 64 * (tq ? 1 : (n + 16 * tt - 1) / (16 * tt)), steps = (cols + 31) / 32;
-    if (ks == 0) {
-        // A wavefront's steps run back to back on its SIMD's f64 matrix core, so a launch wants
-        // EXACT_GEMM_WAVES_PER_CU wavefronts per CU: fewer tiles than that cut K into slices of
-        // at least 8 steps, as many as the workspace holds.
-        ks = 1;
-        const uint64_t want = (uint64_t)EXACT_GEMM_WAVES_PER_CU * g->cus;
-        if (tiles < want && ws) {
-            uint64_t k = std::min<uint64_t>({(want + tiles - 1) / tiles, EXACT_GEMM_MAX_SLICES, steps / 8,
-                                             ws_bytes / (n * rows * 8)});
-            ks = (uint32_t)std::max<uint64_t>(k, 1);
-        }
-    }
-    static const void* const quads[8] = {(const void*)&x0ne_gemm_f64_q1_bf16, (const void*)&x0ne_gemm_f64_q2_bf16,
-                                         (const void*)&x0ne_gemm_f64_q3_bf16, (const void*)&x0ne_gemm_f64_q4_bf16,
-                                         (const void*)&x0ne_gemm_f64_q5_bf16, (const void*)&x0ne_gemm_f64_q6_bf16,
-                                         (const void*)&x0ne_gemm_f64_q7_bf16, (const void*)&x0ne_gemm_f64_q8_bf16};
-    const void* fn = tq ? quads[tq - 1] : (const void*)&x0ne_gemm_f64_t4_bf16;
+    const ExactPlan plan = exact_plan(rows, cols, n, g->cus, ks, ws ? ws_bytes : 0);
+    ks = plan.slices;
+    const void* fn = plan.kind->fn;
     uint32_t r32 = (uint32_t)rows, c32 = (uint32_t)cols, n32 = (uint32_t)n, of = out_f32 ? 1u : 0u, k32 = ks;
     double* wsp = ks > 1 ? ws : nullptr;
     void* yp = y;
@@ -449,7 +486,7 @@ x0ne_status exact_gemm(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols,
                     (void*)&wsp};
     g->counts.gemms++;
     g->counts.launches++;
-    X0NE_HIP(x0ne_launch(fn, dim3((uint32_t)((tiles * ks + 3) / 4)), dim3(256), args, 0, g->stream), "exact gemm");
+    X0NE_HIP(x0ne_launch(fn, dim3((uint32_t)((plan.tiles * ks + 3) / 4)), dim3(256), args, 0, g->stream), "exact gemm");
     if (ks > 1) {
         const double* wsc = wsp;
         void* rargs[] = {(void*)&wsc, (void*)&yp, (void*)&r32, (void*)&n32, (void*)&k32, (void*)&of};
