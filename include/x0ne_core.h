@@ -102,11 +102,13 @@ x0ne_status x0ne_gpu_launch_3d(x0ne_gpu* g, const char* name, uint32_t gx, uint3
 
 /* Gpu::gemm (gpu.rs:1098-1149), the projection the reference hands cuBLAS: Y[n][rows] =
    X[n][cols] W^T, W [rows][cols] row-major bf16, X bf16, f32 accumulation; out_f32 = 0 gives
-   bf16 Y, 1 f32 Y. Device addresses. One row of X: the bandwidth-bound GEMV; 2 to 64 rows (cols
-   a multiple of 8, W and X each below 4 GiB): one few-row matrix-core launch that reads each W
-   row once (x0ne_gemm_few_*); more rows (rows a multiple of 4, 16-byte aligned operands): this
-   library's tiled matrix-core GEMM (x0ne_gpu_gemm_tiled with the tile chosen for the shape);
-   other shapes: one GEMV per row of X. */
+   bf16 Y, 1 f32 Y. Device addresses. One row of X: the bandwidth-bound GEMV; more rows (W's rows a
+   multiple of 4, cols of 8, W and X each below 4 GiB, 16-byte aligned operands): this library's
+   tiled matrix-core GEMM (x0ne_gpu_gemm_tiled with the tile chosen for the shape); a few rows of a
+   small W, and up to 64 rows where W's rows are no multiple of 4: one few-row matrix-core launch
+   (x0ne_gemm_few_*); other shapes: one GEMV per row of X. A shape of few tiles cuts K into slices,
+   whose f32 sums go through a workspace of the Gpu (64 MiB, allocated at its first such call or
+   when a capture begins). The same shape runs the same kernels: the same bits. */
 x0ne_status x0ne_gpu_gemv(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n, uint64_t y,
                           int out_f32);
 /* The tiled matrix-core GEMM of x0ne_gpu_gemv past 64 rows with an explicit block tile (output

@@ -328,10 +328,12 @@ def test_the_tiled_gemm_at_the_prefill_shapes(kernels, name, rows, cols):
 
 
 @pytest.mark.parametrize("rows,cols,n", [(64, 4096, 65), (1000, 2056, 65), (260, 12288, 100), (516, 4104, 200),
-                                         (4096, 4096, 257), (1024, 3072, 777), (2052, 1032, 333), (4, 1024, 65)])
+                                         (4096, 4096, 257), (1024, 3072, 777), (2052, 1032, 333), (4, 1024, 65),
+                                         (4, 2056, 17), (132, 12296, 9), (6148, 4096, 2), (4096, 4096, 9), (4096, 4096, 31),
+                                         (24576, 1024, 64)])
 def test_the_gemm_of_few_tiles_cuts_k_into_slices(kernels, rows, cols, n):
-    """Gpu::gemm past 64 rows where the tiles are too few for the chip: the K slices and their
-    reduction, at ends inside a tile, a stage and a slice. Against float64 products within the
+    """Gpu::gemm past a row where the tiles are too few for the chip: the K slices and their
+    reduction, and the small tiles, at ends inside a tile, a stage and a slice. Against float64 products within the
     GEMV tolerance for f32 sums, the bf16 output the f32 output rounded, the same bits on a
     second call, from panels where W's rows are a multiple of 16, and replayed from a graph."""
     rng = np.random.default_rng(rows + cols + n)
@@ -344,9 +346,12 @@ def test_the_gemm_of_few_tiles_cuts_k_into_slices(kernels, rows, cols, n):
     b = kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, False)
     assert (b == bf16_bits(f).reshape(b.shape)).all()
     assert (kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, True).view(np.uint32) == f.view(np.uint32)).all()
+    t = kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, True, tile=0)
     if rows % 16 == 0:
         p = kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, True, tile=0, layout=W_PANELS | X_PANELS)
-        assert (p.view(np.uint32) == f.view(np.uint32)).all()
+        assert (p.view(np.uint32) == t.view(np.uint32)).all()
+    if n > 16:
+        assert (t.view(np.uint32) == f.view(np.uint32)).all()
     from x0ne_core import Arena, Class
     g, a = kernels.gpu, Arena()
     ws, xs, ys = (a.alloc(k, v, Class.CLIENT_DATA) for k, v in (("w", w.size * 2), ("x", x.size * 2), ("y", n * rows * 4)))

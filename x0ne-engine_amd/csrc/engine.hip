@@ -46,6 +46,7 @@ namespace {
 constexpr uint64_t PREFILL_CHUNK = 2048;
 // The exact mode's prefill GEMM: f64 parts of up to this many bytes (a short pass cuts K into
 // slices to fill the chip).
+constexpr uint32_t FEW_ROWS = 32;
 constexpr uint64_t EXACT_PARTS_BYTES = 64ull << 20;
 constexpr uint64_t MAX_BATCH = 64;  // the few-row GEMM's most rows
 constexpr uint32_t ARGMAX_SLICES = 64;  // blocks per logits row of the batched step's argmax
@@ -515,7 +516,7 @@ uint64_t tile_parts_bytes(const x0ne_engine* e) {
     const uint64_t shapes[4][2] = {{c.qkv_rows(), c.hidden}, {c.hidden, c.q_dim()}, {2 * c.inter, c.hidden}, {c.hidden, c.inter}};
     uint64_t most = 0;
     for (const auto& s : shapes)
-        for (uint64_t n = 65; n <= e->chunk; n += 8) {
+        for (uint64_t n = FEW_ROWS + 1; n <= e->chunk; n += 8) {
             const uint32_t k = x0ne_gemm_tile_plan((uint32_t)s[0], (uint32_t)s[1], (uint32_t)n, e->gpu->cus, TILE_PARTS_BYTES).slices;
             if (k > 1) most = std::max(most, k * n * s[0] * 4);
         }
@@ -972,7 +973,7 @@ x0ne_status gemm(x0ne_engine* e, x0ne_slice w, x0ne_slice w_panels, uint64_t row
     if (!e->ppanel)
         return gemv_rows(e->gpu, (uint64_t)(uintptr_t)e->d(w), rows, cols, (uint64_t)(uintptr_t)e->d(x), n,
                          (uint64_t)(uintptr_t)e->d(y), false, work);
-    if (n <= 64) return skinny(e->gpu, e->d(w_panels), rows, cols, e->d(x), n, e->d(y), 0, PANEL_X | PANEL_W);
+    if (n <= (e->max_batch > 1 ? 64u : FEW_ROWS)) return skinny(e->gpu, e->d(w_panels), rows, cols, e->d(x), n, e->d(y), 0, PANEL_X | PANEL_W);
     return tiled_gemm(e->gpu, 0, X0NE_GEMM_W_PANELS | X0NE_GEMM_X_PANELS, e->d(w_panels), rows, cols, e->d(x), n,
                       e->d(y), false, work);
 }

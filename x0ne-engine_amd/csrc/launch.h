@@ -51,7 +51,14 @@ uint32_t x0ne_gemv_grid(const X0neGemv& g, uint32_t cus, uint32_t max_blocks_per
 // multiple of 16, X's panels hold ceil(n / 16) whole panels). The plan names the block tile
 // (features x tokens) and the K slices (more than one: their f32 sums go through parts,
 // [slices][n][rows]); x0ne_gemm_tile_plan picks both for a shape, within parts_bytes.
-enum { X0NE_TILE_256x256 = 1, X0NE_TILE_256x128 = 2, X0NE_TILE_128x128 = 3, X0NE_TILE_64x64 = 4 };
+enum {
+    X0NE_TILE_256x256 = 1,
+    X0NE_TILE_256x128 = 2,
+    X0NE_TILE_128x128 = 3,
+    X0NE_TILE_64x64 = 4,
+    X0NE_TILE_128x32 = 5,
+    X0NE_TILE_16x16 = 6
+};
 enum { X0NE_TILE_F32 = 1, X0NE_TILE_W_PANEL = 2, X0NE_TILE_X_PANEL = 4 };
 struct X0neTilePlan {
     int tile;

@@ -274,17 +274,18 @@ extern "C" x0ne_status x0ne_gpu_launch_3d(x0ne_gpu* g, const char* name, uint32_
     return launch_checked(g, *k, gx, gy, block, args, n, gz);
 }
 
-// Gpu::gemm (gpu.rs:1098-1149). One row: the bandwidth-bound GEMV of gemv.hip. Two to 64 rows:
-// the few-row kernel of gemm.hip, still bandwidth-bound (each W row read once). More: the tiled
-// matrix-core GEMM. The kernels of gemm.hip take 32-bit buffer offsets.
+// Gpu::gemm (gpu.rs:1098-1149). One row: the bandwidth-bound GEMV of gemv.hip. More: the tiled
+// matrix-core GEMM of gemm.hip; for a few rows of a small W, and up to 64 rows of a shape it does
+// not take, the few-row kernels (still each W row read once); else a GEMV per row. The kernels of gemm.hip take 32-bit buffer
+// offsets.
 static constexpr uint64_t SKINNY_MAX_ROWS = 64;
 static constexpr uint64_t GEMM_MAX_BYTES = 0xFFFFFFF0ull;
 
 namespace x0ne {
 
 // ---- many rows: the tiled matrix-core GEMM of gemm.hip ----
-// The reference hands Gpu::gemm to cuBLAS (gpu.rs:1098-1149); from SKINNY_MAX_ROWS + 1 rows on
-// this library runs its own tiled GEMM (x0ne_launch_gemm_tiles), the tile and the K slices chosen
+// The reference hands Gpu::gemm to cuBLAS (gpu.rs:1098-1149); past one row this library runs its
+// own tiled GEMM (x0ne_launch_gemm_tiles), the tile and the K slices chosen
 // per shape by x0ne_gemm_tile_plan unless `tile` names one (then unsplit). A shape always runs the
 // same kernels, and each output is summed in a fixed order: results are the same from call to
 // call.
@@ -594,7 +595,7 @@ extern "C" x0ne_status x0ne_gpu_gemm_tiled(x0ne_gpu* g, uint32_t tile, uint32_t 
 extern "C" x0ne_status x0ne_gpu_gemv(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n,
                                      uint64_t y, int out_f32) {
     if (!g) return fail(X0NE_ERR_GPU, "no device");
-    return x0ne::gemv_rows(g, w, rows, cols, x, n, y, out_f32 != 0, n > SKINNY_MAX_ROWS ? tile_work(g) : TileWork{});
+    return x0ne::gemv_rows(g, w, rows, cols, x, n, y, out_f32 != 0, n > 1 ? tile_work(g) : TileWork{});
 }
 
 x0ne_status x0ne::gemv_rows(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n, uint64_t y,
@@ -603,15 +604,18 @@ x0ne_status x0ne::gemv_rows(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t col
         return fail(X0NE_ERR_FORMAT, "gemv: " + std::to_string(rows) + "x" + std::to_string(cols) + ", n " +
                                          std::to_string(n));
     const uint64_t ob = out_f32 ? 4 : 2;
+    // A small W by a few rows is over in the time a block takes to start, load and end: there the
+    // few-row kernel, whose wavefronts split K with all their loads in flight, is the faster one
+    // (4096 x 1024 by 8 rows 5.5 against 6.6 us, by 32 level; 4096 x 4096 by 4 10.6 against 11.2, by 16
+    // 12.8 against 11.5; from 50 MB of W on the tiled GEMM at every count: 6144 x 4096 by 2 15.4
+    // against 14.0).
+    const bool small = 2 * rows * cols < 40'000'000 && n <= (cols <= 2048 ? 16u : 8u);
+    if (n >= 2 && !small && cols % 8 == 0 && rows % 4 == 0 && n <= UINT32_MAX && rows * cols * 2 <= GEMM_MAX_BYTES &&
+        n * cols * 2 <= GEMM_MAX_BYTES && w % 16 == 0 && x % 16 == 0 && y % 16 == 0)
+        return x0ne::tiled_gemm(g, 0, 0, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32, work);
     if (n >= 2 && n <= SKINNY_MAX_ROWS && cols % 8 == 0 && rows * cols * 2 <= GEMM_MAX_BYTES && w % 16 == 0 &&
         x % 16 == 0)
         return x0ne::skinny(g, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32 ? 1 : 0, 0);
-    // Many rows: the tiled matrix-core GEMM (rows a multiple of 4, aligned operands; otherwise the
-    // row-by-row GEMV below).
-    if (n > SKINNY_MAX_ROWS && cols % 8 == 0 && rows % 4 == 0 && n <= UINT32_MAX &&
-        rows * cols * 2 <= GEMM_MAX_BYTES && n * cols * 2 <= GEMM_MAX_BYTES && w % 16 == 0 && x % 16 == 0 &&
-        y % 16 == 0)
-        return x0ne::tiled_gemm(g, 0, 0, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32, work);
     for (uint64_t r = 0; r < n; ++r) {
         const uint16_t* wp = (const uint16_t*)w;
         const uint16_t* xp = (const uint16_t*)(x + r * cols * 2);
