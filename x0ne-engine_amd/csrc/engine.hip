@@ -942,8 +942,15 @@ x0ne_status feed(x0ne_engine* e, uint32_t i) {
     return run_step(e);
 }
 
-x0ne_status put_prompt(x0ne_engine* e, const uint32_t* ids, size_t n) {
-    return x0ne_arena_write(e->arena, e->prompt, 0, ids, n * 4);
+// Sequence b's prompt ids. Not waited for: the work that reads them is queued behind the copy, and
+// every entry point that takes ids drains the stream, on success and on failure, before it
+// returns them to the caller.
+x0ne_status put_prompt(x0ne_engine* e, const uint32_t* ids, size_t n, uint64_t b = 0) {
+    uint64_t off;
+    X0NE_TRY(arena_check(e->arena, e->prompt, b * e->max_ctx * 4, n * 4, &off));
+    e->gpu->counts.htod++;
+    X0NE_HIP(hipMemcpyAsync(e->arena->base + off, ids, n * 4, hipMemcpyHostToDevice, e->gpu->stream), "prompt");
+    return X0NE_OK;
 }
 
 // Sequence b's token = its prompt[i], its position = i, without a step.
@@ -2120,7 +2127,7 @@ x0ne_status batch_checks(x0ne_engine* e, const uint32_t* prompts, size_t np, siz
 x0ne_status batch_prefill(x0ne_engine* e, const uint32_t* prompts, size_t np, uint32_t B, size_t n, uint32_t* tokens) {
     if (e->mode == X0NE_DECODE_GRAPH) X0NE_TRY(batch_capture(e, B));
     for (uint32_t b = 0; b < B; ++b)
-        X0NE_TRY(x0ne_arena_write(e->arena, e->prompt, (uint64_t)b * e->max_ctx * 4, prompts + (size_t)b * np, np * 4));
+        X0NE_TRY(put_prompt(e, prompts + (size_t)b * np, np, b));
     // Prompts that fit a pass several at a time go together (chunk / np of them; with panels np
     // a multiple of 16), the others one sequence at a time in passes of up to chunk rows. Only
     // prompts of more than 64 rows: a sequence alone then runs the same tiled GEMM as the shared
