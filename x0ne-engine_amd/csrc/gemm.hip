@@ -630,9 +630,10 @@ extern "C" __global__ void __launch_bounds__(256)
 //    LDS, filled by direct buffer-to-LDS loads (buffer_load_dwordx4 ... lds: no registers, no
 //    VALU) issued STAGES stages ahead. One barrier per stage.
 //  - The operands of each 32-column step are read from LDS into a second register set while the
-//    products of the step before run, the reads interleaved with the products (one read, then
-//    products), so the matrix cores do not wait for LDS. Measured on MI355X (Qwen3-8B shapes,
-//    2048 rows): 0.4-0.47 of bf16 peak against 0.36-0.43 without the overlap.
+//    products of the step before run, and the next stage's loads are issued among them, one read
+//    or load between every few products, so the matrix cores wait for neither: 2048 x 24576 x 4096
+//    317 us (1.30 PFLOP/s; a library product of that shape 322), x 6144 x 4096 95 (87), x 4096 x
+//    12288 173 (175), x 4096 x 4096 64 (61).
 //  - LDS holds 16 rows x 64 columns of an operand as 2 KiB, the two fragments (16 rows x 32 k)
 //    that the products read; either layout is read without bank conflicts (256 bytes per clock,
 //    measured on gfx950). Operands in 16-row panels (device.h: [rows / 16][cols / 8][16][8]): a
@@ -687,16 +688,16 @@ __device__ __forceinline__ i32x4 rsrc_words(const void* base, uint64_t bytes) {
 }
 
 // One direct buffer-to-LDS load (buffer_load_dwordx4 ... lds): lane l's 16 bytes at byte offset
-// `off` of the buffer (zeros past it) land at LDS byte lds + 16 l. Written as an instruction of
+// off + soff of the buffer (zeros past it) land at LDS byte lds + 16 l. Written as an instruction of
 // its own so the compiler adds no wait of its own for it: the loop below counts these loads and
 // waits for them itself. M0 holds the LDS address; nothing else in these kernels uses M0.
-__device__ __forceinline__ void load_lds16(const i32x4& r, uint32_t lds, uint32_t off) {
-    // The descriptor and the LDS address are wavefront-uniform; read from lane 0 so they are
+__device__ __forceinline__ void load_lds16(const i32x4& r, uint32_t lds, uint32_t off, uint32_t soff) {
+    // The descriptor, the LDS address and soff are wavefront-uniform; read from lane 0 so they are
     // scalar registers whatever the compiler concluded.
     const i32x4 u = {__builtin_amdgcn_readfirstlane(r[0]), __builtin_amdgcn_readfirstlane(r[1]),
                      __builtin_amdgcn_readfirstlane(r[2]), __builtin_amdgcn_readfirstlane(r[3])};
-    asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dwordx4 %0, %2, 0 offen lds" ::"v"(off),
-                 "s"(__builtin_amdgcn_readfirstlane(lds)), "s"(u)
+    asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dwordx4 %0, %2, %3 offen lds" ::"v"(off),
+                 "s"(__builtin_amdgcn_readfirstlane(lds)), "s"(u), "s"(__builtin_amdgcn_readfirstlane(soff))
                  : "memory");
 }
 
@@ -738,11 +739,10 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
 
     // This wavefront's loads of a stage: load h (0, 1) of 16-row group g = wave + NW (q / 2) (W's
     // groups first). In panels lane l fetches row l % 16, columns 32 h + 8 (l / 16) .. + 7 of the
-    // stage; row-major, row 8 h + l / 8, columns 8 ((l % 8) ^ (l / 8)) .. + 7: byte
-    // base[q] + step[q] s of the buffer while those columns exist and the row (panel: its group
-    // of 16) does.
-    uint32_t base[C::LOADS], step[C::LOADS], chunk0[C::LOADS];
-    bool row_in[C::LOADS];
+    // stage; row-major, row 8 h + l / 8, columns 8 ((l % 8) ^ (l / 8)) .. + 7. A lane's offset in
+    // its operand is voff[q] (past the buffer for a row that does not exist) and, the same for
+    // every lane, w_step or x_step per stage; a stage that reaches past cols checks its columns.
+    uint32_t voff[C::LOADS], chunk0[C::LOADS];
 #pragma unroll
     for (int q = 0; q < C::LOADS; ++q) {
         const int h = q % TILE_K, g = (int)wave + C::NW * (q / TILE_K);
@@ -750,20 +750,20 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
         const uint32_t g16 = ((is_w ? f0 : t0) >> 4) + (uint32_t)(is_w ? g : g - C::WFR);
         const bool panel = is_w ? w_panel : x_panel;
         const uint32_t row = 16 * g16 + (panel ? 0 : 8 * h + (lane >> 3));
-        row_in[q] = row < (is_w ? rows : n);
-        step[q] = TILE_K * (panel ? 1024 : 64);
         chunk0[q] = panel ? 4 * h + (lane >> 4) : (lane & 7) ^ (lane >> 3);
-        base[q] = (panel ? g16 * c8 * 256 + 1024 * h + 16 * lane : row * cols * 2 + 16 * chunk0[q]) + step[q] * first;
-        chunk0[q] += 4 * TILE_K * first;
+        voff[q] = row >= (is_w ? rows : n) ? OFF_NONE
+                  : panel                  ? g16 * c8 * 256 + 1024 * h + 16 * lane
+                                           : row * cols * 2 + 16 * chunk0[q];
     }
-    auto issue = [&](uint32_t s) {
-        uint8_t* dst = lds + (s % STAGES) * C::BYTES;
-#pragma unroll
-        for (int q = 0; q < C::LOADS; ++q) {
-            const int h = q % TILE_K, g = (int)wave + C::NW * (q / TILE_K);
-            const bool in = row_in[q] && 4 * TILE_K * s + chunk0[q] < c8;
-            load_lds16(g < C::WFR ? wr : xr, lds_addr(dst + g * C::GROUP + h * 1024), in ? base[q] + step[q] * s : OFF_NONE);
-        }
+    const uint32_t w_step = TILE_K * (w_panel ? 1024 : 64), x_step = TILE_K * (x_panel ? 1024 : 64);
+    const uint32_t lds0 = lds_addr(lds) + wave * C::GROUP;
+    auto load = [&](uint32_t s, int q) {
+        const int h = q % TILE_K, g = C::NW * (q / TILE_K);
+        const bool is_w = (int)wave + g < C::WFR;
+        uint32_t off = voff[q];
+        if (4 * TILE_K * (first + s + 1) > c8 && 4 * TILE_K * (first + s) + chunk0[q] >= c8) off = OFF_NONE;
+        load_lds16(is_w ? wr : xr, lds0 + (s % STAGES) * C::BYTES + g * C::GROUP + h * 1024, off,
+                   (first + s) * (is_w ? w_step : x_step));
     };
 
     f32x4 acc[C::RA][C::RB];
@@ -788,20 +788,31 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
 #pragma unroll
         for (int j = 0; j < C::RB; ++j) bx[j] = *reinterpret_cast<const uint4*>(src + x_at[kk] + j * C::GROUP);
     };
-    // The products of one stage, with the reads issued just before them interleaved: one LDS
-    // read, then its share of the products.
-    auto compute = [&](const uint4 (&a)[C::RA], const uint4 (&bx)[C::RB]) {
-#pragma unroll
-        for (int i = 0; i < C::RA; ++i)
-#pragma unroll
-            for (int j = 0; j < C::RB; ++j) acc[i][j] = mfma(a[i], bx[j], acc[i][j]);
+    // One step: the products of (a, bx); among them, evenly, the reads of the next step's operands
+    // (step kk of stage s) into (na, nb) and, with LOAD, the loads of stage ls. The order is as
+    // written: the loads in one run in front of the products left the matrix cores idle for it
+    // (2048 x 24576 x 4096 346 -> 317 us; in the first half of the step 333).
+    auto step = [&](const uint4 (&a)[C::RA], const uint4 (&bx)[C::RB], uint32_t s, int kk, uint4 (&na)[C::RA],
+                    uint4 (&nb)[C::RB], bool loads, uint32_t ls) {
+        const uint8_t* src = lds + (s % STAGES) * C::BYTES;
         constexpr int R = C::RA + C::RB, M = C::RA * C::RB;
+        int m = 0;
 #pragma unroll
-        for (int i = 0; i < R; ++i) {
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // one LDS read
-            __builtin_amdgcn_sched_group_barrier(0x008, M / R, 0);  // then products
+        for (int g = 0; g < R; ++g) {
+            if (loads)
+#pragma unroll
+                for (int q = g * C::LOADS / R; q < (g + 1) * C::LOADS / R; ++q) load(ls, q);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (; m < (g + 1) * M / R; ++m)
+                acc[m / C::RB][m % C::RB] = mfma(a[m / C::RB], bx[m % C::RB], acc[m / C::RB][m % C::RB]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (g < C::RA)
+                na[g] = *reinterpret_cast<const uint4*>(src + w_at[kk] + g * C::GROUP);
+            else
+                nb[g - C::RA] = *reinterpret_cast<const uint4*>(src + x_at[kk] + (g - C::RA) * C::GROUP);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        if (M % R) __builtin_amdgcn_sched_group_barrier(0x008, M % R, 0);
     };
 
     // Prologue: stages 0 .. STAGES - 1 in flight, stage 0 complete (this wavefront's loads: at
@@ -809,7 +820,10 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
     // operands read.
 #pragma unroll
     for (int p = 0; p < STAGES; ++p)
-        if ((uint32_t)p < stages) issue(p);
+        if ((uint32_t)p < stages) {
+#pragma unroll
+            for (int q = 0; q < C::LOADS; ++q) load(p, q);
+        }
     if (stages >= (uint32_t)STAGES) {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::LOADS * (STAGES - 1)) : "memory");
     } else {
@@ -817,46 +831,34 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
     }
     asm volatile("s_barrier" ::: "memory");
     read(0, 0, a0, b0);
-    // Step kk of stage s: its products run while the next step's operands are read. Before the
-    // last step of stage s: stage s + 1 complete in this wavefront (at most min(stages - s - 2,
-    // STAGES - 2) later stages' loads in flight) and its own reads of stage s done; the barrier:
-    // the same in every wavefront, so stage s's slot is no longer read and takes stage
-    // s + STAGES. The next step after the last one reads stage s's last step again (a harmless
-    // read that keeps the reads unconditional). The two steps of a stage alternate between the
-    // register sets. (Two stages per turn of the loop: with one, the compiler moves the 256 x 256
-    // tile's accumulators between registers and the kernel takes twice the time.)
-    for (uint32_t s2 = 0; s2 < stages; s2 += 2) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const uint32_t s = s2 + h;
-            if (s >= stages) break;
-#pragma unroll
-            for (int kk = 0; kk < TILE_K; ++kk) {
-                uint32_t ns = s;
-                int nk = kk + 1;
-                if (kk == TILE_K - 1) {
-                    if (s + 1 < stages) {
-                        if (stages - s - 2 >= (uint32_t)(STAGES - 2)) {
-                            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::LOADS * (STAGES - 2)) : "memory");
-                        } else {
-                            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-                        }
-                    }
-                    __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
-                    asm volatile("s_barrier" ::: "memory");
-                    if (s + STAGES < stages) issue(s + STAGES);
-                    ns = s + 1 < stages ? s + 1 : s;
-                    nk = s + 1 < stages ? 0 : kk;
-                }
-                if (kk % 2 == 0) {
-                    read(ns, nk, a1, b1);
-                    compute(a0, b0);
-                } else {
-                    read(ns, nk, a0, b0);
-                    compute(a1, b1);
-                }
+    // The two steps of stage s alternate between the register sets; each step's products run while
+    // the next step's operands are read. Before its last step: stage s + 1 complete in this
+    // wavefront (at most min(stages - s - 2, STAGES - 2) later stages' loads in flight) and its own
+    // reads of stage s done; the barrier: the same in every wavefront, so stage s's slot is no
+    // longer read and takes stage s + STAGES. The last step's reads fetch stage s's again (harmless,
+    // they keep the reads unconditional).
+    auto turn = [&](uint32_t s) {
+        if (s + 1 < stages) {
+            if (stages - s - 2 >= (uint32_t)(STAGES - 2)) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::LOADS * (STAGES - 2)) : "memory");
+            } else {
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             }
         }
+        __builtin_amdgcn_s_waitcnt(WAIT_LGKM0);
+        asm volatile("s_barrier" ::: "memory");
+    };
+    static_assert(TILE_K == 2, "two steps per stage");
+    uint32_t s = 0;
+    for (; s + STAGES < stages; ++s) {
+        step(a0, b0, s, 1, a1, b1, false, 0);
+        turn(s);
+        step(a1, b1, s + 1, 0, a0, b0, true, s + STAGES);
+    }
+    for (; s < stages; ++s) {
+        step(a0, b0, s, 1, a1, b1, false, 0);
+        turn(s);
+        step(a1, b1, s + 1 < stages ? s + 1 : s, 0, a0, b0, false, 0);
     }
 
     // acc[i][j][r]: feature f0 + WF wf + 16 i + 4 (lane / 16) + r, token t0 + WT wt + 16 j + lane % 16.

@@ -605,11 +605,13 @@ x0ne_status x0ne::gemv_rows(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t col
                                          std::to_string(n));
     const uint64_t ob = out_f32 ? 4 : 2;
     // A small W by a few rows is over in the time a block takes to start, load and end: there the
-    // few-row kernel, whose wavefronts split K with all their loads in flight, is the faster one
-    // (4096 x 1024 by 8 rows 5.5 against 6.6 us, by 32 level; 4096 x 4096 by 4 10.6 against 11.2, by 16
-    // 12.8 against 11.5; from 50 MB of W on the tiled GEMM at every count: 6144 x 4096 by 2 15.4
-    // against 14.0).
-    const bool small = 2 * rows * cols < 40'000'000 && n <= (cols <= 2048 ? 16u : 8u);
+    // few-row kernel, whose wavefronts split K with all their loads in flight, is the faster one, for
+    // as many rows as its steps are few (us, few-row against tiled: 4096 x 1024 by 8 rows 5.5 / 6.6,
+    // by 32 6.7 / 6.9, by 48 8.4 / 7.0; 6144 x 1024, two blocks on some CUs, by 16 6.5 / 6.7, by 24
+    // 7.4 / 6.9; 4096 x 4096 by 4 10.6 / 11.2, by 16 12.8 / 11.5). From 50 MB of W on the tiled GEMM at
+    // every count: 6144 x 4096 by 2 15.4 / 14.0.
+    const uint64_t few = cols > 2048 ? 8 : cols > 1024 || rows > 16ull * g->cus ? 16 : 32;
+    const bool small = 2 * rows * cols < 40'000'000 && n <= few;
     if (n >= 2 && !small && cols % 8 == 0 && rows % 4 == 0 && n <= UINT32_MAX && rows * cols * 2 <= GEMM_MAX_BYTES &&
         n * cols * 2 <= GEMM_MAX_BYTES && w % 16 == 0 && x % 16 == 0 && y % 16 == 0)
         return x0ne::tiled_gemm(g, 0, 0, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32, work);
