@@ -291,8 +291,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void* base, u
 
 // The default cache policy: a non-temporal hint on the K/V tiles measured no faster at short
 // contexts and 12 % slower at 32k keys on MI355X.
-__device__ __forceinline__ uint4 bload16(__amdgpu_buffer_rsrc_t r, uint32_t off) {
-    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0);
+__device__ __forceinline__ uint4 bload16(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t uniform_off = 0) {
+    const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)uniform_off, 0);
     return make_uint4((uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]);
 }
 // One word through the vector memory path: a page-table entry fetched ahead this way is waited
@@ -1393,13 +1393,13 @@ __device__ __forceinline__ void attn_group_block(const AttnArgs& a, AttnShared<G
 // ([rows][q_heads][128] bf16, at positions pos0 + row): its 128 columns (column c: row
 // r0 + c / G, head kh G + c % G) go 32 to a wavefront, as two groups of 16 (the 16 columns of a
 // product). The keys pass in tiles of 64 (4 pages) staged in LDS once per block and read by all
-// 4 wavefronts (K [64][128], V dim-major [128][64], chunks swizzled against bank conflicts);
+// 4 wavefronts (K by products, V dim-major, chunks swizzled against bank conflicts);
 // each K or V piece a wavefront reads serves both groups.
 // Per tile and column group: S^T = K Q^T (16 products; the S^T blocks X0, Y0, X1, Y1 of the
 // decode wavefront, which leave each lane the 8 keys of its P row for a 32-key step), a
 // per-column causal mask (keys up to the column's own position; skipped for a tile inside every
-// limit of the wavefront), the online softmax in units of log2 (the rescale of O skipped when no
-// maximum of the group moved), and O += P V with P rounded to bf16 (16 products). The next
+// limit of the wavefront), the online softmax in units of log2 (O rescaled only when a column's
+// maximum passed its reference by 2^8), and O += P V with P rounded to bf16 (16 products). The next
 // tile's loads are in flight while a tile is multiplied (two LDS buffers). Each column's output
 // goes straight to out ([rows][q_heads][128], or in 16-row panels). The heavier half of the row blocks is dispatched
 // first, heaviest first, then the lighter half, lightest first. Keys at or past the block's context are read as zeros (V) or masked (K); no page past
@@ -1413,23 +1413,27 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
 constexpr int PF_CG = 2;              // column groups of 16 per wavefront
 constexpr int PF_NW = X0NE_PREFILL_THREADS / 64;  // wavefronts per block
 static_assert(PF_NW * 16 * PF_CG == X0NE_PREFILL_COLS, "columns per prefill block");
-// LDS tiles without padding: K [64 keys][128 dims], V [128 dims][64 keys], their 16-byte chunks
-// placed by an XOR of the row (pf_k_chunk, pf_v_chunk) so that neither the products' reads nor
-// the stores of a tile meet in a bank. Measured on gfx950 (bank-conflict counters over single
-// access patterns): 16-byte reads are served 16 lanes at a time (lanes that differ in bits 0, 1,
-// 3 and 4 of the lane id) over 128 four-byte banks, 16-byte writes 8 neighbouring lanes at a
-// time over 32 banks.
-constexpr uint32_t PF_KS = 128;  // bf16 per K row in LDS
-constexpr uint32_t PF_VS = 64;   // bf16 per V dim row in LDS
-// Chunk slot of 16-byte chunk c (dims 8 c ..) of K row r, and of chunk c (keys 8 c ..) of V row d.
-__device__ __forceinline__ uint32_t pf_k_chunk(uint32_t r, uint32_t c) {
-    return c ^ (2 * ((r >> 1) & 1) + 4 * ((r >> 3) & 1) + 8 * ((r >> 4) & 1));
+constexpr float PF_LAZY = 8.f;
+// LDS tiles without padding, in KiB of 8 rows x 128 bytes whose 16-byte chunks are placed by an XOR
+// of the row, so that the 16 rows x 4 chunks that a product's operand reads meet in no bank (gfx950:
+// 256 bytes per clock, measured over single access patterns) and neither do 8 neighbouring lanes'
+// stores. The layout before, by rows of the tile, spent 38 % of the LDS cycles in conflicts.
+// K: the keys of a product's 16 rows together: block (kp, h) holds keys 32 kp + 8 a + 4 h + j as rows
+// n = 4 a + j, dims 0..63 in front of 64..127. V: row = dim, 64 keys of 2 bytes.
+// Element index of 16-byte chunk c (dims 8 c ..) of key r, and of chunk c (keys 8 c ..) of dim d.
+__device__ __forceinline__ uint32_t pf_chunk(uint32_t row, uint32_t c) {
+    return ((row >> 3) * 64 + (row & 7) * 8 + (c ^ (row & 7))) * 8;
 }
-__device__ __forceinline__ uint32_t pf_v_chunk(uint32_t d, uint32_t c) { return c ^ (2 * ((d >> 2) & 3)); }
+__device__ __forceinline__ uint32_t pf_k_at(uint32_t kp, uint32_t h, uint32_t n, uint32_t c) {
+    return ((kp * 2 + h) * 2 + (c >> 3)) * 1024 + pf_chunk(n, c & 7);
+}
+__device__ __forceinline__ uint32_t pf_k_key(uint32_t r, uint32_t c) {
+    return pf_k_at(r >> 5, (r >> 2) & 1, 4 * ((r >> 3) & 3) + (r & 3), c);
+}
 
 struct PrefillShared {
-    alignas(16) bf16_t k[2][X0NE_SPLIT_TILE * PF_KS];
-    alignas(16) bf16_t v[2][X0NE_HEAD_DIM * PF_VS];
+    alignas(1024) bf16_t k[2][X0NE_SPLIT_TILE * X0NE_HEAD_DIM];
+    alignas(1024) bf16_t v[2][X0NE_HEAD_DIM * X0NE_SPLIT_TILE];
 };
 
 template <int G, int CG, bool OUT_PANEL = false, int NW = 4>
@@ -1474,30 +1478,30 @@ __device__ __forceinline__ void prefill_block(const bf16_t* __restrict__ q, cons
     // A tile's K and V pieces for this thread: K chunk i = t + NT j is page i / 256, key
     // (i / 16) % 16, 16-byte piece i % 16; V chunk i is page i / 256, dim v_dim(i), keys
     // 8 (i % 2) .. + 7 of the page. A wavefront's V loads cover 32 dims of a page (1 KiB
-    // contiguous), and 8 neighbouring lanes hold dims 4 apart, so their LDS chunks differ.
-    // Their loads are issued by fetch() and waited for only by stash(), after a tile's products.
-    // The page-table entries of a tile are requested one tile before its K and V.
-    auto v_dim = [](uint32_t i) { return 32 * ((i >> 6) & 3) + 16 * ((i >> 5) & 1) + 4 * ((i >> 1) & 3) + ((i >> 3) & 3); };
+    // contiguous), and 8 neighbouring lanes hold dims 2 apart, so their LDS chunks differ.
+    // Their loads are issued by fetch() and waited for only by stash(), after a tile's products. The
+    // thread's chunk j of a tile is in the tile's page j: its page-table entry is the same for the
+    // whole block, so it is a scalar, requested one tile before the K and V (an entry past the
+    // context is the last one again: those keys are masked), and a load's address is a lane's constant
+    // plus a scalar.
+    static_assert(NT == 256 && J == X0NE_SPLIT_TILE / X0NE_PAGE, "chunk j of a thread is in page j of the tile");
+    auto v_dim = [](uint32_t i) { return 32 * ((i >> 6) & 3) + 8 * ((i >> 4) & 3) + 2 * ((i >> 1) & 3) + ((i >> 3) & 1); };
     auto v_half = [](uint32_t i) { return i & 1; };
     uint4 kr[J], vr[J];
     const auto kres = plane_rsrc(k_cache, OFF_NONE), vres = plane_rsrc(v_cache, OFF_NONE);
-    uint32_t pe[J];  // entries of the next tile to fetch (chunk j of a thread is in page (t + NT j) / 256)
+    const uint32_t k_lane = (((t >> 4) & 15) * X0NE_HEAD_DIM + 8 * (t & 15)) * 2;
+    const uint32_t v_lane = (v_dim(t) * X0NE_PAGE + 8 * v_half(t)) * 2;
+    uint32_t pe[J];  // entries of the next tile to fetch
     auto entries = [&](uint32_t tile) {
 #pragma unroll
-        for (int j = 0; j < (int)J; ++j) {
-            const uint32_t pi = (t + NT * j) >> 8;
-            pe[j] = 4 * tile + pi < npages ? pages[4 * tile + pi] : 0u;
-        }
+        for (int j = 0; j < (int)J; ++j) pe[j] = pages[min(4 * tile + j, npages - 1)];
     };
     auto fetch = [&](uint32_t tile) {
 #pragma unroll
         for (int j = 0; j < (int)J; ++j) {
-            const uint32_t i = t + NT * j, pi = i >> 8, lp = 4 * tile + pi;
-            const uint32_t pb = pe[j] * kv_heads + kh;
-            kr[j] = bload16(kres, lp < npages ? ((pb * X0NE_PAGE + ((i >> 4) & 15)) * X0NE_HEAD_DIM + 8 * (i & 15)) * 2
-                                              : OFF_NONE);
-            vr[j] = bload16(vres, lp < npages ? ((pb * X0NE_HEAD_DIM + v_dim(i)) * X0NE_PAGE + 8 * v_half(i)) * 2
-                                              : OFF_NONE);
+            const uint32_t at = __builtin_amdgcn_readfirstlane((pe[j] * kv_heads + kh) * (X0NE_PAGE * X0NE_HEAD_DIM * 2));
+            kr[j] = bload16(kres, k_lane, at);
+            vr[j] = bload16(vres, v_lane, at);
         }
     };
     auto stash = [&](uint32_t tile, int buf) {
@@ -1520,8 +1524,8 @@ __device__ __forceinline__ void prefill_block(const bf16_t* __restrict__ q, cons
 #pragma unroll
         for (int j = 0; j < (int)J; ++j) {
             const uint32_t i = t + NT * j, pi = i >> 8, r = 16 * pi + ((i >> 4) & 15), d = v_dim(i);
-            *reinterpret_cast<uint4*>(&sh.k[buf][r * PF_KS + 8 * pf_k_chunk(r, i & 15)]) = kr[j];
-            *reinterpret_cast<uint4*>(&sh.v[buf][d * PF_VS + 8 * pf_v_chunk(d, 2 * pi + v_half(i))]) = vr[j];
+            *reinterpret_cast<uint4*>(&sh.k[buf][pf_k_key(r, i & 15)]) = kr[j];
+            *reinterpret_cast<uint4*>(&sh.v[buf][pf_chunk(d, 2 * pi + v_half(i))]) = vr[j];
         }
     };
 
@@ -1564,13 +1568,12 @@ __device__ __forceinline__ void prefill_block(const bf16_t* __restrict__ q, cons
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 // A row n: key 32 kp + 8 (n >> 2) + 4 h + (n & 3)
-                const uint32_t row = 32 * kp + 8 * (n >> 2) + 4 * h + (n & 3);
                 f32x4 acc[CG];
 #pragma unroll
                 for (int cg = 0; cg < CG; ++cg) acc[cg] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int st = 0; st < 4; ++st) {
-                    const uint4 kk = *reinterpret_cast<const uint4*>(K + row * PF_KS + 8 * pf_k_chunk(row, 4 * st + q4));
+                    const uint4 kk = *reinterpret_cast<const uint4*>(K + pf_k_at(kp, h, n, 4 * st + q4));
 #pragma unroll
                     for (int cg = 0; cg < CG; ++cg) acc[cg] = mfma16x16x32(kk, qb[cg][st], acc[cg]);
                 }
@@ -1607,8 +1610,12 @@ __device__ __forceinline__ void prefill_block(const bf16_t* __restrict__ q, cons
 #pragma unroll
                     for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[cg][kp][h][i]);
             mx = rows_max(mx);
+            // The column's reference moves when its maximum passes it by more than 2^PF_LAZY: weights
+            // up to 2^PF_LAZY keep their relative precision in bf16 and f32, and O and l are seldom
+            // rescaled (some column of 16 has a new maximum in most of a prompt's first tiles).
             // Key 0 is in every column's first tile, so m_run is finite from there on.
-            const float mn = fmaxf(m_run[cg], mx * scale2);
+            const float top = mx * scale2;
+            const float mn = top > m_run[cg] + PF_LAZY ? top : m_run[cg];
             const float alpha = __builtin_amdgcn_exp2f(m_run[cg] - mn);
             m_run[cg] = mn;
             float sc[2][2][4];
@@ -1623,7 +1630,7 @@ __device__ __forceinline__ void prefill_block(const bf16_t* __restrict__ q, cons
                         psum += sc[kp][h][i];
                     }
             lsum[cg] = lsum[cg] * alpha + psum;
-            if (__any(alpha != 1.f)) {  // multiplying by 1 changes nothing: skipped when no max moved
+            if (__any(alpha != 1.f)) {  // multiplying by 1 changes nothing: skipped when none moved
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float ai = __shfl(alpha, 4 * q4 + i, 64);
@@ -1651,7 +1658,7 @@ __device__ __forceinline__ void prefill_block(const bf16_t* __restrict__ q, cons
 #pragma unroll
             for (int nb = 0; nb < 8; ++nb) {
                 const uint32_t d = 16 * nb + n;
-                const uint4 vb = *reinterpret_cast<const uint4*>(V + d * PF_VS + 8 * pf_v_chunk(d, 4 * kp + q4));
+                const uint4 vb = *reinterpret_cast<const uint4*>(V + pf_chunk(d, 4 * kp + q4));
 #pragma unroll
                 for (int cg = 0; cg < CG; ++cg) o[cg][nb] = mfma16x16x32(phi[cg][kp], vb, o[cg][nb]);
             }
