@@ -1398,8 +1398,8 @@ __device__ __forceinline__ void attn_group_block(const AttnArgs& a, AttnShared<G
 // Per tile and column group: S^T = K Q^T (16 products; the S^T blocks X0, Y0, X1, Y1 of the
 // decode wavefront, which leave each lane the 8 keys of its P row for a 32-key step), a
 // per-column causal mask (keys up to the column's own position; skipped for a tile inside every
-// limit of the wavefront), the online softmax in units of log2 (O rescaled only when a column's
-// maximum passed its reference by 2^8), and O += P V with P rounded to bf16 (16 products). The next
+// limit of the wavefront), the online softmax in units of log2 (the rescale of O skipped when no
+// maximum of the group moved), and O += P V with P rounded to bf16 (16 products). The next
 // tile's loads are in flight while a tile is multiplied (two LDS buffers). Each column's output
 // goes straight to out ([rows][q_heads][128], or in 16-row panels). The heavier half of the row blocks is dispatched
 // first, heaviest first, then the lighter half, lightest first. Keys at or past the block's context are read as zeros (V) or masked (K); no page past
@@ -1413,7 +1413,6 @@ __device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
 constexpr int PF_CG = 2;              // column groups of 16 per wavefront
 constexpr int PF_NW = X0NE_PREFILL_THREADS / 64;  // wavefronts per block
 static_assert(PF_NW * 16 * PF_CG == X0NE_PREFILL_COLS, "columns per prefill block");
-constexpr float PF_LAZY = 8.f;
 // LDS tiles without padding, in KiB of 8 rows x 128 bytes whose 16-byte chunks are placed by an XOR
 // of the row, so that the 16 rows x 4 chunks that a product's operand reads meet in no bank (gfx950:
 // 256 bytes per clock, measured over single access patterns) and neither do 8 neighbouring lanes'
@@ -1610,12 +1609,8 @@ __device__ __forceinline__ void prefill_block(const bf16_t* __restrict__ q, cons
 #pragma unroll
                     for (int i = 0; i < 4; ++i) mx = fmaxf(mx, s[cg][kp][h][i]);
             mx = rows_max(mx);
-            // The column's reference moves when its maximum passes it by more than 2^PF_LAZY: weights
-            // up to 2^PF_LAZY keep their relative precision in bf16 and f32, and O and l are seldom
-            // rescaled (some column of 16 has a new maximum in most of a prompt's first tiles).
             // Key 0 is in every column's first tile, so m_run is finite from there on.
-            const float top = mx * scale2;
-            const float mn = top > m_run[cg] + PF_LAZY ? top : m_run[cg];
+            const float mn = fmaxf(m_run[cg], mx * scale2);
             const float alpha = __builtin_amdgcn_exp2f(m_run[cg] - mn);
             m_run[cg] = mn;
             float sc[2][2][4];
@@ -1630,7 +1625,7 @@ __device__ __forceinline__ void prefill_block(const bf16_t* __restrict__ q, cons
                         psum += sc[kp][h][i];
                     }
             lsum[cg] = lsum[cg] * alpha + psum;
-            if (__any(alpha != 1.f)) {  // multiplying by 1 changes nothing: skipped when none moved
+            if (__any(alpha != 1.f)) {  // multiplying by 1 changes nothing: skipped when no max moved
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const float ai = __shfl(alpha, 4 * q4 + i, 64);
