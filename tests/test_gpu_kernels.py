@@ -366,6 +366,53 @@ def test_the_gemm_of_few_tiles_cuts_k_into_slices(kernels, rows, cols, n):
         assert (a.read_array(ys, 0, n * rows, np.uint32) == f.view(np.uint32).ravel()).all()
 
 
+def test_a_gpu_takes_its_slices_workspace_while_another_thread_captures(kernels):
+    """The first call that cuts K into slices allocates the Gpu's workspace: made in one thread while
+    another holds a capture of its own Gpu open, it neither fails, nor ends the capture, nor goes
+    unsplit (the bits of a Gpu that took its workspace outside any capture)."""
+    import threading
+
+    from x0ne_core import Arena, Class, Gpu
+    rows, cols, n = 516, 4104, 200
+    rng = np.random.default_rng(5)
+    w, x = (bf16_bits(O.bf16_round(rng.normal(0, s, k).astype(np.float32))) for s, k in ((0.02, rows * cols), (1.0, n * cols)))
+
+    def inputs(gpu):
+        a, sl = Arena(), {}
+        for name, size in (("w", w.size * 2), ("x", x.size * 2), ("y", n * rows * 4)):
+            sl[name] = a.alloc(name, size, Class.CLIENT_DATA)
+        a.freeze(gpu)
+        a.write(sl["w"], 0, w)
+        a.write(sl["x"], 0, x)
+        return a, sl["y"], lambda: gpu.gemv(a.ptr(sl["w"]), rows, cols, a.ptr(sl["x"]), n, a.ptr(sl["y"]), True)
+
+    fresh = Gpu()
+    a, y, call = inputs(kernels.gpu)
+    b, by, fresh_call = inputs(fresh)
+    errors = []
+
+    def other():
+        try:
+            fresh_call()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    def captured():
+        call()
+        t = threading.Thread(target=other)
+        t.start()
+        t.join()
+
+    graph = kernels.gpu.capture(captured)
+    assert not errors, errors
+    kernels.gpu.launch_graph(graph)
+    kernels.gpu.sync()
+    fresh.sync()
+    got = a.read_array(y, 0, n * rows, np.uint32)
+    assert (got == b.read_array(by, 0, n * rows, np.uint32)).all()
+    assert (got == kernels.gemm(w, rows, cols, x, n, True).view(np.uint32).ravel()).all()
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_few_row_gemm_is_the_oracle_and_its_swiglu_the_swiglu_kernel(kernels, seed):
     """The batched step's projection kernel (2 to 64 rows of X, each W row read once) at every

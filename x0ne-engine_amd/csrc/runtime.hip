@@ -276,8 +276,8 @@ extern "C" x0ne_status x0ne_gpu_launch_3d(x0ne_gpu* g, const char* name, uint32_
 
 // Gpu::gemm (gpu.rs:1098-1149). One row: the bandwidth-bound GEMV of gemv.hip. More: the tiled
 // matrix-core GEMM of gemm.hip; for a few rows of a small W, and up to 64 rows of a shape it does
-// not take, the few-row kernels (still each W row read once); else a GEMV per row. The kernels of gemm.hip take 32-bit buffer
-// offsets.
+// not take, the few-row kernels (still each W row read once); else a GEMV per row. The kernels of
+// gemm.hip take 32-bit buffer offsets.
 static constexpr uint64_t SKINNY_MAX_ROWS = 64;
 static constexpr uint64_t GEMM_MAX_BYTES = 0xFFFFFFF0ull;
 
@@ -317,11 +317,16 @@ x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, ui
 // GEMMs stay unsplit.
 static TileWork tile_work(x0ne_gpu* g) {
     if (!g->tile_parts && !g->tile_parts_refused && !g->capturing) {
+        // Another thread may have a capture of its own Gpu open: this thread's mode is relaxed for the
+        // allocation, so that it is neither refused nor ends that capture.
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
         if (hipMalloc((void**)&g->tile_parts, TILE_PARTS_BYTES) != hipSuccess) {
             (void)hipGetLastError();
             g->tile_parts = nullptr;
             g->tile_parts_refused = true;
         }
+        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
     }
     return g->tile_parts ? TileWork{g->tile_parts, TILE_PARTS_BYTES} : TileWork{};
 }
