@@ -920,6 +920,32 @@ def test_the_isolated_attention_timing_rotates_distinct_planes(kernels):
         assert us > 0 and planes >= 2 and 2 * plane * planes > 512 << 20, (ctx, p, us, planes)
 
 
+@pytest.mark.parametrize("seed", range(2))
+def test_swiglu_of_every_gate_is_the_f64_value_rounded(kernels, seed):
+    """Eight values at a time (f32 first, f64 where that is not sure to round alike) against single
+    values (a length that is no multiple of 8: f64 for each): the same bits for all 65536 gates with
+    48 ups, among them zeros, the ends of the exponents, infinities and NaN; and numpy's f64 value."""
+    rng = np.random.default_rng(seed)
+    ups = np.concatenate([np.array([0, 0x8000, 1, 0x007F, 0x0080, 0x3F80, 0xBF80, 0x7F7F, 0xFF7F, 0x7F80, 0xFF80, 0x7FC0], np.uint16),
+                          bf16_bits(O.bf16_round(rng.normal(0, 1, 20).astype(np.float32))),
+                          rng.integers(0, 1 << 16, 16).astype(np.uint16)])
+    gates = rng.permutation(1 << 16).astype(np.uint16)
+    gu = np.stack([np.stack([gates, np.full(1 << 16, u, np.uint16)]) for u in ups])
+    fast = kernels.swiglu_rows(gu.ravel(), len(ups)).reshape(len(ups), -1)
+    padded = np.concatenate([gu, np.zeros((len(ups), 2, 1), np.uint16)], -1)
+    single = kernels.swiglu_rows(padded.ravel(), len(ups)).reshape(len(ups), -1)[:, :-1]
+    assert (fast == single).all(), f"{(fast != single).sum()} of {fast.size} differ"
+    panel = kernels.swiglu_rows(gu.ravel(), len(ups), panel=True).reshape(len(ups), -1)
+    assert (panel == single).all()
+    with np.errstate(all="ignore"):
+        g, u = (bf16_vals(gu[:, i].ravel()).astype(np.float64).reshape(len(ups), -1) for i in (0, 1))
+        want = (g / (1.0 + np.exp(-g)) * u).astype(np.float32)
+    assert (np.isnan(want) == np.isnan(bf16_vals(fast.ravel()).reshape(want.shape))).all()
+    ok = np.isfinite(want)
+    same = bf16_bits(O.bf16_round(np.where(ok, want, 0).astype(np.float32).ravel())).reshape(want.shape) == fast
+    assert (same | ~ok).mean() > 0.99999  # numpy's exponential may differ in its last place
+
+
 @pytest.mark.parametrize("seed", range(20))
 def test_swiglu_is_the_oracle(kernels, seed):
     rng = O.Rng(600 + seed)

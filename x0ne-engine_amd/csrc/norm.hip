@@ -205,10 +205,14 @@ extern "C" __global__ void __launch_bounds__(256)
 // x0ne_add_rmsnorm_bf16 with out in panels (hidden a multiple of 8): the batched step's norms,
 // whose rows feed the few-row GEMM. The same bits at the panel positions (a chunk of 8 values is
 // 8 consecutive panel elements). grid (rows), block 256.
+// Blocks go round the 8 XCDs, and a cache line of a panel holds pieces of 8 rows: of every 128 rows the
+// blocks of one XCD take the same 16, so that a line is written whole from one L2 (2048 rows of 4096:
+// 26.0 -> 20.0 us).
 extern "C" __global__ void __launch_bounds__(256)
     x0ne_add_rmsnorm_panel_bf16(float* __restrict__ residual, const bf16_t* __restrict__ x,
                                 const bf16_t* __restrict__ w, bf16_t* __restrict__ out, uint32_t hidden, float eps) {
-    const uint32_t row = blockIdx.x;
+    const uint32_t b = blockIdx.x, r128 = b & ~127u;
+    const uint32_t row = r128 + 128 <= gridDim.x ? r128 + 16 * (b & 7) + ((b & 127) >> 3) : b;
     const size_t base = (size_t)row * hidden;
     float* res = residual + base;
     const bf16_t* xr = x + base;
@@ -364,13 +368,53 @@ extern "C" __global__ void __launch_bounds__(256)
     cs[2 * k + 1] = sin(angle);
 }
 
-// SwiGLU on the packed [gate; up] row: out[i] = g / (1 + e^-g) * u, in f64 (swiglu.cu:5-11;
-// oracle/src/lib.rs:205-214). Thread t of block x takes values 8 (256 x + t) .. + 7 of row y:
-// 16-byte loads of gate and up and one 16-byte store where inter is a multiple of 8 and both
+// SwiGLU on the packed [gate; up] row: out[i] = bf16(f32(g / (1 + e^-g) * u)) of the f64 value
+// (swiglu.cu:5-11; oracle/src/lib.rs:205-214). Thread t of block x takes values 8 (256 x + t) .. + 7
+// of row y: 16-byte loads of gate and up and one 16-byte store where inter is a multiple of 8 and both
 // pointers are 16-byte aligned (single values otherwise). grid (ceil(inter / 2048), rows), block 256.
+// Every value's f64 exponential and division took longer than its 6 bytes. The value is computed in
+// f32 first, and in f64 only where the f32 error reaches a rounding boundary of bf16 (Ziv's rounding
+// test), about one value in 1,500: the same bits (333 rows of 24576 in the L2: 8.8 -> 6.5 us).
 __device__ __forceinline__ bf16_t swiglu1(bf16_t g16, bf16_t u16) {
     const double g = (double)bf2f(g16), u = (double)bf2f(u16);
     return f2bf((float)(g / (1.0 + exp(-g)) * u));
+}
+// The f32 value's bf16, and whether it is surely swiglu1's. For |g| < 64, x = -g log2(e) is one
+// rounding of its exact sum (g's 8 bits times 15 of the constant's, and the rest), so e^-g is off by
+// |g| 2^-24 of itself plus the exponential's ulp; with the sum, the reciprocal (1 ulp) and the two
+// products the value is off by less than 2^-21 + |g| 2^-24, that is by 8 + |g| units of its last
+// place. Twice that is kept from the middle between two bf16 values (the low half word at 0x8000);
+// rounding is monotonic, so the f64 value lands on the same one. Zeros, the far ends of the exponents,
+// infinities and NaN are not sure.
+__device__ __forceinline__ bf16_t swiglu_f32(bf16_t g16, bf16_t u16, bool& sure) {
+    const float g = bf2f(g16), u = bf2f(u16), a = fabsf(g);
+    const float e = __builtin_amdgcn_exp2f(fmaf(-g, 7.0526076e-06f, -g * 1.44268798828125f));
+    const float v = g * __builtin_amdgcn_rcpf(1.0f + e) * u;
+    const uint32_t b = __float_as_uint(v), mag = b & 0x7FFFFFFFu;
+    const int off = abs((int)(b & 0xFFFFu) - 0x8000);
+    sure = a < 64.0f && mag > 0x0D800000u && mag < 0x72000000u && off > 18 + (int)(2.0f * a);  // 2^-100 .. 2^101
+    return f2bf(v);
+}
+// Eight values from 16-byte aligned gate and up into 16 bytes at o, the first one's place; those that
+// are not sure are stored a second time.
+__device__ __forceinline__ void swiglu8(const bf16_t* gate, const bf16_t* up, bf16_t* o) {
+    const uint4 g = *reinterpret_cast<const uint4*>(gate), u = *reinterpret_cast<const uint4*>(up);
+    const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
+    uint32_t ow[4], again = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        bool lo, hi;
+        ow[j] = (uint32_t)swiglu_f32((bf16_t)(gw[j] & 0xFFFFu), (bf16_t)(uw[j] & 0xFFFFu), lo);
+        ow[j] |= (uint32_t)swiglu_f32((bf16_t)(gw[j] >> 16), (bf16_t)(uw[j] >> 16), hi) << 16;
+        again |= (lo ? 0u : 1u << (2 * j)) | (hi ? 0u : 2u << (2 * j));
+    }
+    *reinterpret_cast<uint4*>(o) = make_uint4(ow[0], ow[1], ow[2], ow[3]);
+    for (; again; again &= again - 1) {
+        const int k = __builtin_ctz(again), j = k >> 1, sh = 16 * (k & 1);
+        const uint32_t gk = j == 0 ? gw[0] : j == 1 ? gw[1] : j == 2 ? gw[2] : gw[3];
+        const uint32_t uk = j == 0 ? uw[0] : j == 1 ? uw[1] : j == 2 ? uw[2] : uw[3];
+        o[k] = swiglu1((bf16_t)(gk >> sh), (bf16_t)(uk >> sh));
+    }
 }
 extern "C" __global__ void __launch_bounds__(256)
     x0ne_swiglu_bf16(const bf16_t* __restrict__ gate_up, bf16_t* __restrict__ out, uint32_t inter) {
@@ -379,38 +423,28 @@ extern "C" __global__ void __launch_bounds__(256)
     const bf16_t* row = gate_up + (size_t)r * 2 * inter;
     bf16_t* o = out + (size_t)r * inter;
     if (inter % 8 == 0 && (((uintptr_t)gate_up | (uintptr_t)out) & 15) == 0) {  // grid-uniform
-        const uint4 g = *reinterpret_cast<const uint4*>(row + i0);
-        const uint4 u = *reinterpret_cast<const uint4*>(row + inter + i0);
-        const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
-        uint32_t ow[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            ow[j] = (uint32_t)swiglu1((bf16_t)(gw[j] & 0xFFFFu), (bf16_t)(uw[j] & 0xFFFFu)) |
-                    ((uint32_t)swiglu1((bf16_t)(gw[j] >> 16), (bf16_t)(uw[j] >> 16)) << 16);
-        *reinterpret_cast<uint4*>(o + i0) = make_uint4(ow[0], ow[1], ow[2], ow[3]);
+        swiglu8(row + i0, row + inter + i0, o + i0);
         return;
     }
     for (uint32_t i = i0; i < min(i0 + 8, inter); ++i) o[i] = swiglu1(row[i], row[inter + i]);
 }
 
 // x0ne_swiglu_bf16 with out in 16-row panels (device.h) of inter columns, for the prefill pass's
-// down projection: the same values (swiglu1 of each gate and up pair), stored at panel_index.
-// grid (ceil(inter / 2048), rows), block 256.
+// down projection: the same values, stored at panel_index. grid (ceil(inter / 2048), rows), block 256.
+// A row's 16-byte pieces lie 256 bytes apart in a panel, eighths of cache lines that 8 blocks, each on
+// another XCD, would write. Eight blocks that follow one another in y share their 8 rows out by columns
+// instead: a wavefront reads 8 rows x 128 bytes and writes 8 lines of 8 rows x 16 bytes (2048 rows of
+// 24576: 57 -> 25.5 us, 5.9 TB/s). The rows past the last whole 8 go one per block.
 extern "C" __global__ void __launch_bounds__(256)
     x0ne_swiglu_panel_bf16(const bf16_t* __restrict__ gate_up, bf16_t* __restrict__ out, uint32_t inter) {
-    const uint32_t i0 = 8 * (blockIdx.x * blockDim.x + threadIdx.x), r = blockIdx.y;
+    const uint32_t t = threadIdx.x, r8 = blockIdx.y & ~7u;
+    const bool eight = blockDim.x == 256 && r8 + 8 <= gridDim.y;
+    const uint32_t i0 = 8 * (blockIdx.x * blockDim.x + (eight ? 32 * (blockIdx.y & 7) + (t >> 3) : t));
+    const uint32_t r = eight ? r8 + (t & 7) : blockIdx.y;
     if (i0 >= inter) return;
     const bf16_t* row = gate_up + (size_t)r * 2 * inter;
     if (inter % 8 == 0 && ((uintptr_t)gate_up & 15) == 0 && ((uintptr_t)out & 15) == 0) {  // grid-uniform
-        const uint4 g = *reinterpret_cast<const uint4*>(row + i0);
-        const uint4 u = *reinterpret_cast<const uint4*>(row + inter + i0);
-        const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
-        uint32_t ow[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-            ow[j] = (uint32_t)swiglu1((bf16_t)(gw[j] & 0xFFFFu), (bf16_t)(uw[j] & 0xFFFFu)) |
-                    ((uint32_t)swiglu1((bf16_t)(gw[j] >> 16), (bf16_t)(uw[j] >> 16)) << 16);
-        *reinterpret_cast<uint4*>(out + panel_index(r, i0, inter)) = make_uint4(ow[0], ow[1], ow[2], ow[3]);
+        swiglu8(row + i0, row + inter + i0, out + panel_index(r, i0, inter));
         return;
     }
     for (uint32_t i = i0; i < min(i0 + 8, inter); ++i) out[panel_index(r, i, inter)] = swiglu1(row[i], row[inter + i]);
