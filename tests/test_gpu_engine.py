@@ -200,6 +200,24 @@ def test_greedy_on_the_device_is_greedy_on_the_host(which):
         print(f"MEASURE greedy prompt {prompt_len}: compared {compared} of {n} tokens with the oracle")
 
 
+@pytest.mark.parametrize("q_heads,kv_heads", [(2, 2), (4, 2), (8, 2), (8, 1)])
+@pytest.mark.parametrize("np_,batch,chunk", [(65, 5, 0), (77, 5, 176), (95, 2, 0), (96, 3, 192), (113, 4, 2048)])
+def test_prompts_of_any_length_share_a_pass_and_keep_their_bits(q_heads, kv_heads, np_, batch, chunk):
+    """Prompts of more than 64 ids go through a pass together, each sequence's rows at the next multiple
+    of 16 (77 ids in passes of 176 rows: two at a time, the fifth alone), QK-norm + RoPE and the attention
+    of all of them in one launch each: tokens and last logits are the bits each sequence gets alone."""
+    from x0ne_core import Engine, EngineOptions
+    f = Fixture(tiny(2, q_heads, kv_heads, False), 23)
+    e = Engine.load_from(f.cfg.to_json(), {"model.safetensors": f.file},
+                         EngineOptions(max_ctx=128, page_seed=4, prefill_chunk=chunk, max_batch=5))
+    prompts = np.stack([f.tokens(500 + b, np_) for b in range(batch)])
+    toks, _, logits = e.greedy_batch(prompts, 4, logits=True)
+    assert e.client_data_is_zero()
+    for b in range(batch):
+        t1, _, l1 = e.greedy_batch(prompts[b:b + 1], 4, logits=True)
+        assert (t1[0] == toks[b]).all() and (l1[0].view(np.uint32) == logits[b].view(np.uint32)).all(), f"sequence {b}"
+
+
 @pytest.mark.parametrize("which,np_,chunk", [(0, 21, 16), (1, 21, 16), (0, 80, 0), (1, 80, 0)])
 def test_batched_greedy_is_each_sequence_alone_and_the_oracle(which, np_, chunk):
     """B independent prompts decoded together (the batched step: few-row GEMMs, one attention

@@ -1711,6 +1711,23 @@ __device__ __forceinline__ void prefill_block(const bf16_t* __restrict__ q, cons
         __shared__ PrefillShared sh;                                                                               \
         prefill_block<G, PF_CG, true, PF_NW>(q, k_cache, v_cache, pages, out, pos0[0], rows, q_heads, kv_heads,      \
                                              max_ctx, scale, sh);                                                  \
+    }                                                                                                              \
+    /* The panel kernel over several sequences of `rows` rows, one per blockIdx.z: sequence s has the   */          \
+    /* rows from s stride on of q and out (stride a multiple of 16: whole panels), pos0[s] and the      */          \
+    /* seq_pages page-table entries from s seq_pages on. 512 rows of one sequence are 128 blocks for    */          \
+    /* 512 places on the chip; four sequences fill them in one launch.                                  */          \
+    extern "C" __global__ void __launch_bounds__(X0NE_PREFILL_THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) \
+        x0ne_attention_prefill_seqs_g##G##_bf16(                                                                  \
+        const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,    \
+        const uint32_t* __restrict__ pages, bf16_t* __restrict__ out, const uint32_t* __restrict__ pos0,          \
+        uint32_t rows, uint32_t q_heads, uint32_t kv_heads, uint32_t max_ctx, float scale, uint32_t stride,         \
+        uint32_t seq_pages) {                                                                                      \
+        __shared__ PrefillShared sh;                                                                               \
+        const size_t at = (size_t)blockIdx.z * stride * q_heads * X0NE_HEAD_DIM;                                   \
+        if (stride % 16 != 0) return;                                                                              \
+        prefill_block<G, PF_CG, true, PF_NW>(q + at, k_cache, v_cache, pages + (size_t)blockIdx.z * seq_pages,     \
+                                             out + at, pos0[blockIdx.z], rows, q_heads, kv_heads, max_ctx, scale,  \
+                                             sh);                                                                  \
     }
 X0NE_PREFILL_GROUP(1)
 X0NE_PREFILL_GROUP(2)

@@ -993,19 +993,22 @@ x0ne_status gemm(x0ne_engine* e, x0ne_slice w, x0ne_slice w_panels, uint64_t row
 // prompt row, position and KV pages. With ppanel the GEMM inputs are written in panels (the same
 // values at panel_index) and the GEMMs read W's panel copies.
 // seqs > 1 (a batched engine's prompts of one length): sequences b .. b + seqs - 1 in one pass,
-// n rows each at the same positions, side by side (rows s n .. s n + n - 1 are sequence b + s):
-// the GEMMs, norms and SwiGLU take all seqs n rows at once, QK-norm + RoPE and the attention run
-// per sequence on its rows, pages and position. With panels n is a multiple of 16, so each
-// sequence's rows start a panel.
+// n rows each at the same positions, side by side (sequence b + s's rows start at s pass_rows(n)):
+// the GEMMs, norms and SwiGLU take all rows at once, QK-norm + RoPE and the attention each
+// sequence's n rows with its pages and position (one launch with panels, else one per sequence). With
+// panels each sequence's rows start a panel; the rows between are token 0's, and no output of another
+// row depends on them.
+uint64_t pass_rows(const x0ne_engine* e, uint64_t n) { return e->ppanel ? (n + 15) / 16 * 16 : n; }
+
 x0ne_status prefill_pass(x0ne_engine* e, uint64_t pos0, uint64_t n, uint64_t b = 0, uint64_t seqs = 1) {
     const Cfg& c = e->c;
-    if (e->chunk < 2 || n == 0 || seqs == 0 || n * seqs > e->chunk || pos0 + n > e->max_ctx || b + seqs > e->max_batch ||
-        (seqs > 1 && e->ppanel && n % 16 != 0))
+    const uint64_t stride = seqs > 1 ? pass_rows(e, n) : n;
+    if (e->chunk < 2 || n == 0 || seqs == 0 || stride * seqs > e->chunk || pos0 + n > e->max_ctx || b + seqs > e->max_batch)
         return fail(X0NE_ERR_FORMAT, "prefill: " + std::to_string(seqs) + " x " + std::to_string(n) + " rows at " +
                                          std::to_string(pos0));
     for (uint64_t s = 0; s < seqs; ++s) X0NE_TRY(set_position(e, pos0, b + s));
-    const uint32_t sn = (uint32_t)n;  // rows of one sequence
-    n *= seqs;
+    const uint32_t sn = (uint32_t)n, st = (uint32_t)stride;  // rows of one sequence, and to the next one's
+    n = stride * seqs;
     const uint32_t rows = (uint32_t)n, h = (uint32_t)c.hidden, vocab = (uint32_t)c.vocab, inter = (uint32_t)c.inter;
     const uint32_t qh = (uint32_t)c.q_heads, kvh = (uint32_t)c.kv_heads, max_ctx = (uint32_t)e->max_ctx;
     const float eps = (float)c.eps, scale = (float)(1.0 / std::sqrt((double)c.head_dim));
@@ -1013,8 +1016,12 @@ x0ne_status prefill_pass(x0ne_engine* e, uint64_t pos0, uint64_t n, uint64_t b =
         const void* table = e->d(e->embed);
         const void* toks = e->prompt_of(b) + pos0;
         if (seqs > 1) {  // the sequences' ids of this pass side by side
+            if (st != sn) {
+                e->gpu->counts.memsets++;
+                X0NE_HIP(hipMemsetAsync(e->d(e->p_tok), 0, n * 4, e->gpu->stream), "pass ids");
+            }
             e->gpu->counts.launches++;
-            X0NE_HIP(hipMemcpy2DAsync(e->d(e->p_tok), (size_t)sn * 4, toks, e->max_ctx * 4, (size_t)sn * 4, seqs,
+            X0NE_HIP(hipMemcpy2DAsync(e->d(e->p_tok), (size_t)st * 4, toks, e->max_ctx * 4, (size_t)sn * 4, seqs,
                                       hipMemcpyDeviceToDevice, e->gpu->stream),
                      "pass ids");
             toks = e->d(e->p_tok);
@@ -1036,6 +1043,14 @@ x0ne_status prefill_pass(x0ne_engine* e, uint64_t pos0, uint64_t n, uint64_t b =
     };
     const uint32_t group = qh / kvh;
     const bool pp = e->ppanel;
+    // One launch for all sequences of a pass (panels, so 1, 2, 4 or 8 q heads per kv head).
+    const bool together = seqs > 1 && pp;
+    const uint32_t runs = together ? 1 : (uint32_t)seqs, z = together ? (uint32_t)seqs : 1;
+    const uint32_t seq_pages = (uint32_t)e->seq_pages;
+    const void* seqs_fn = group == 1   ? (const void*)&x0ne_attention_prefill_seqs_g1_bf16
+                          : group == 2 ? (const void*)&x0ne_attention_prefill_seqs_g2_bf16
+                          : group == 4 ? (const void*)&x0ne_attention_prefill_seqs_g4_bf16
+                                       : (const void*)&x0ne_attention_prefill_seqs_g8_bf16;
     const void* grouped = group == 1   ? (pp ? (const void*)&x0ne_attention_prefill_panel_g1_bf16 : (const void*)&x0ne_attention_prefill_g1_bf16)
                           : group == 2 ? (pp ? (const void*)&x0ne_attention_prefill_panel_g2_bf16 : (const void*)&x0ne_attention_prefill_g2_bf16)
                           : group == 4 ? (pp ? (const void*)&x0ne_attention_prefill_panel_g4_bf16 : (const void*)&x0ne_attention_prefill_g4_bf16)
@@ -1052,38 +1067,41 @@ x0ne_status prefill_pass(x0ne_engine* e, uint64_t pos0, uint64_t n, uint64_t b =
         const LayerW& w = e->L[l];
         X0NE_TRY(norm(w.input_norm));
         X0NE_TRY(gemm(e, w.qkv, w.qkv_p, c.qkv_rows(), c.hidden, e->p_x, n, e->p_qkv));
-        for (uint64_t sq = 0; sq < seqs; ++sq) {
-            const void* qkv = e->d(e->p_qkv) + sq * sn * c.qkv_rows() * 2;
+        for (uint64_t sq = 0; sq < runs; ++sq) {
+            const void* qkv = e->d(e->p_qkv) + sq * st * c.qkv_rows() * 2;
             const void* qn = e->d(w.q_norm);
             const void* kn = e->d(w.k_norm);
             const void* cs = e->d(e->rope_cs);
-            void* q = e->d(e->p_q) + sq * sn * c.q_dim() * 2;
+            void* q = e->d(e->p_q) + sq * st * c.q_dim() * 2;
             void* kc = e->plane(l, 0);
             void* vc = e->plane(l, 1);
             const void* pt = e->pages_of(b + sq);
             const void* pos = e->pos_of(b + sq);
             void* args[] = {(void*)&qkv, (void*)&qn, (void*)&kn, (void*)&cs, (void*)&q,       (void*)&kc, (void*)&vc,
-                            (void*)&pt,  (void*)&pos, (void*)&qh, (void*)&kvh, (void*)&max_ctx, (void*)&eps};
-            X0NE_TRY(launch_rows(e, (const void*)&x0ne_qk_norm_rope_kv_write_rows_bf16, dim3((qh + kvh + 3) / 4, sn),
-                                 dim3(256), args, "qk_norm_rope_kv_write"));
+                            (void*)&pt,  (void*)&pos, (void*)&qh, (void*)&kvh, (void*)&max_ctx, (void*)&eps,
+                            (void*)&st,  (void*)&seq_pages};  // the last two: _seqs only
+            X0NE_TRY(launch_rows(e, together ? (const void*)&x0ne_qk_norm_rope_kv_write_seqs_bf16
+                                             : (const void*)&x0ne_qk_norm_rope_kv_write_rows_bf16,
+                                 dim3((qh + kvh + 3) / 4, sn, z), dim3(256), args, "qk_norm_rope_kv_write"));
         }
-        for (uint64_t sq = 0; sq < seqs; ++sq) {
-            const void* q = e->d(e->p_q) + sq * sn * c.q_dim() * 2;
+        for (uint64_t sq = 0; sq < runs; ++sq) {
+            const void* q = e->d(e->p_q) + sq * st * c.q_dim() * 2;
             const void* kc = e->plane(l, 0);
             const void* vc = e->plane(l, 1);
             const void* pt = e->pages_of(b + sq);
-            void* out = e->d(e->p_attn) + sq * sn * c.q_dim() * 2;  // a whole number of panels
+            void* out = e->d(e->p_attn) + sq * st * c.q_dim() * 2;  // a whole number of panels
             const void* pos = e->pos_of(b + sq);
             void* args[] = {(void*)&q,  (void*)&kc, (void*)&vc,  (void*)&pt,      (void*)&out, (void*)&pos,
-                            (void*)&sn, (void*)&qh, (void*)&kvh, (void*)&max_ctx, (void*)&scale};
+                            (void*)&sn, (void*)&qh, (void*)&kvh, (void*)&max_ctx, (void*)&scale,
+                            (void*)&st, (void*)&seq_pages};  // the last two: _seqs only
             if (e->f64_sums) {
                 const uint32_t per = X0NE_PREFILL_EXACT_COLS / group;  // rows per block
                 X0NE_TRY(launch_rows(e, exact, dim3(kvh, (sn + per - 1) / per), dim3(X0NE_PREFILL_EXACT_THREADS), args,
                                      "exact prefill attention"));
             } else if (grouped) {
                 const uint32_t per = X0NE_PREFILL_COLS / group;  // rows per block
-                X0NE_TRY(launch_rows(e, grouped, dim3(kvh, (sn + per - 1) / per), dim3(X0NE_PREFILL_THREADS), args,
-                                     "prefill attention"));
+                X0NE_TRY(launch_rows(e, together ? seqs_fn : grouped, dim3(kvh, (sn + per - 1) / per, z),
+                                     dim3(X0NE_PREFILL_THREADS), args, "prefill attention"));
             } else {
                 X0NE_TRY(launch_rows(e, (const void*)&x0ne_attention_prefill_bf16, dim3(qh, sn), dim3(256), args,
                                      "prefill attention"));
@@ -2128,13 +2146,13 @@ x0ne_status batch_prefill(x0ne_engine* e, const uint32_t* prompts, size_t np, ui
     if (e->mode == X0NE_DECODE_GRAPH) X0NE_TRY(batch_capture(e, B));
     for (uint32_t b = 0; b < B; ++b)
         X0NE_TRY(put_prompt(e, prompts + (size_t)b * np, np, b));
-    // Prompts that fit a pass several at a time go together (chunk / np of them; with panels np
-    // a multiple of 16), the others one sequence at a time in passes of up to chunk rows. Only
+    // Prompts that fit a pass several at a time go together (chunk / pass_rows(np) of them), the
+    // others one sequence at a time in passes of up to chunk rows. Only
     // prompts of more than 64 rows: a sequence alone then runs the same tiled GEMM as the shared
     // pass (64 rows or fewer take the few-row kernel), so each sequence's bits do not depend on
     // the batch.
     const uint64_t per_pass =
-        np > 64 && np <= e->chunk && (!e->ppanel || np % 16 == 0) ? e->chunk / np : 1;
+        np > 64 && np <= e->chunk ? std::max<uint64_t>(e->chunk / pass_rows(e, np), 1) : 1;
     // Its logits row where the batched step leaves the others' (the last token's logits of a
     // one-token request).
     auto keep_logits = [&](uint32_t b) -> x0ne_status {
@@ -2148,7 +2166,7 @@ x0ne_status batch_prefill(x0ne_engine* e, const uint32_t* prompts, size_t np, ui
             const uint32_t seqs = (uint32_t)std::min<uint64_t>(per_pass, B - b);
             X0NE_TRY(prefill_pass(e, 0, np, b, seqs));
             for (uint32_t s = 0; s < seqs; ++s) {
-                X0NE_TRY(prefill_head(e, (uint64_t)s * np + np - 1, np - 1, true, b + s));
+                X0NE_TRY(prefill_head(e, s * (seqs > 1 ? pass_rows(e, np) : np) + np - 1, np - 1, true, b + s));
                 X0NE_TRY(keep_logits(b + s));
             }
             b += seqs;

@@ -24,6 +24,11 @@ __global__ void x0ne_qk_norm_rope_kv_write_rows_bf16(const bf16_t* qkv, const bf
                                                      const double* cs, bf16_t* q_out, bf16_t* k_cache,
                                                      bf16_t* v_cache, const uint32_t* pages, const uint32_t* pos0,
                                                      uint32_t q_heads, uint32_t kv_heads, uint32_t max_ctx, float eps);
+__global__ void x0ne_qk_norm_rope_kv_write_seqs_bf16(const bf16_t* qkv, const bf16_t* q_norm, const bf16_t* k_norm,
+                                                     const double* cs, bf16_t* q_out, bf16_t* k_cache,
+                                                     bf16_t* v_cache, const uint32_t* pages, const uint32_t* pos0,
+                                                     uint32_t q_heads, uint32_t kv_heads, uint32_t max_ctx, float eps,
+                                                     uint32_t stride, uint32_t seq_pages);
 __global__ void x0ne_attention_decode_bf16(const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache,
                                            const uint32_t* pages, bf16_t* out, const uint32_t* pos, uint32_t q_heads,
                                            uint32_t kv_heads, uint32_t max_ctx, float scale);
@@ -74,7 +79,11 @@ __global__ void x0ne_rope_table_f64(const float* inv_freq, double* cs, uint32_t 
                                                       uint32_t max_ctx, float scale);                    \
     __global__ void x0ne_attention_prefill_panel_g##G##_bf16(                                                    \
         const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache, const uint32_t* pages, bf16_t* out,       \
-        const uint32_t* pos0, uint32_t rows, uint32_t q_heads, uint32_t kv_heads, uint32_t max_ctx, float scale);
+        const uint32_t* pos0, uint32_t rows, uint32_t q_heads, uint32_t kv_heads, uint32_t max_ctx, float scale); \
+    __global__ void x0ne_attention_prefill_seqs_g##G##_bf16(                                                     \
+        const bf16_t* q, const bf16_t* k_cache, const bf16_t* v_cache, const uint32_t* pages, bf16_t* out,       \
+        const uint32_t* pos0, uint32_t rows, uint32_t q_heads, uint32_t kv_heads, uint32_t max_ctx, float scale, \
+        uint32_t stride, uint32_t seq_pages);
 X0NE_DECLARE_PREFILL_GROUP(1)
 X0NE_DECLARE_PREFILL_GROUP(2)
 X0NE_DECLARE_PREFILL_GROUP(4)

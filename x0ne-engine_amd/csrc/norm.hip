@@ -312,13 +312,12 @@ extern "C" __global__ void __launch_bounds__(64)
 // positions < max_ctx) instead of computed, and four heads of one row per 256-thread block (one
 // per wavefront). The table holds the f64 values the direct kernel computes, so the two give
 // the same bits. grid (ceil((q_heads + kv_heads) / 4), rows), block 256.
-extern "C" __global__ void __launch_bounds__(256)
-    x0ne_qk_norm_rope_kv_write_rows_bf16(const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ q_norm,
-                                         const bf16_t* __restrict__ k_norm, const double* __restrict__ cs,
-                                         bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache,
-                                         bf16_t* __restrict__ v_cache, const uint32_t* __restrict__ pages,
-                                         const uint32_t* __restrict__ pos0, uint32_t q_heads, uint32_t kv_heads,
-                                         uint32_t max_ctx, float eps) {
+__device__ __forceinline__ void qk_norm_rope_row(const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ q_norm,
+                                                 const bf16_t* __restrict__ k_norm, const double* __restrict__ cs,
+                                                 bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache,
+                                                 bf16_t* __restrict__ v_cache, const uint32_t* __restrict__ pages,
+                                                 const uint32_t* __restrict__ pos0, uint32_t q_heads,
+                                                 uint32_t kv_heads, uint32_t max_ctx, float eps) {
     constexpr uint32_t HD = X0NE_HEAD_DIM, HALF = HD / 2;
     const uint32_t head = blockIdx.x * 4 + (threadIdx.x >> 6), row = blockIdx.y, i = threadIdx.x & 63;
     if (head >= q_heads + kv_heads) return;  // wavefront-uniform
@@ -352,6 +351,29 @@ extern "C" __global__ void __launch_bounds__(256)
     const uint32_t vat = v_slot(pages, pos, kh, kv_heads);
     v_cache[vat + i * X0NE_PAGE] = vs[i];
     v_cache[vat + (i + HALF) * X0NE_PAGE] = vs[i + HALF];
+}
+extern "C" __global__ void __launch_bounds__(256)
+    x0ne_qk_norm_rope_kv_write_rows_bf16(const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ q_norm,
+                                         const bf16_t* __restrict__ k_norm, const double* __restrict__ cs,
+                                         bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache,
+                                         bf16_t* __restrict__ v_cache, const uint32_t* __restrict__ pages,
+                                         const uint32_t* __restrict__ pos0, uint32_t q_heads, uint32_t kv_heads,
+                                         uint32_t max_ctx, float eps) {
+    qk_norm_rope_row(qkv, q_norm, k_norm, cs, q_out, k_cache, v_cache, pages, pos0, q_heads, kv_heads, max_ctx, eps);
+}
+// The same for several sequences, one per blockIdx.z: sequence s has the rows from s stride on of qkv
+// and q_out, pos0[s] and the seq_pages page-table entries from s seq_pages on.
+extern "C" __global__ void __launch_bounds__(256)
+    x0ne_qk_norm_rope_kv_write_seqs_bf16(const bf16_t* __restrict__ qkv, const bf16_t* __restrict__ q_norm,
+                                         const bf16_t* __restrict__ k_norm, const double* __restrict__ cs,
+                                         bf16_t* __restrict__ q_out, bf16_t* __restrict__ k_cache,
+                                         bf16_t* __restrict__ v_cache, const uint32_t* __restrict__ pages,
+                                         const uint32_t* __restrict__ pos0, uint32_t q_heads, uint32_t kv_heads,
+                                         uint32_t max_ctx, float eps, uint32_t stride, uint32_t seq_pages) {
+    const size_t s = blockIdx.z, row0 = s * stride;
+    qk_norm_rope_row(qkv + row0 * (q_heads + 2 * kv_heads) * X0NE_HEAD_DIM, q_norm, k_norm, cs,
+                     q_out + row0 * q_heads * X0NE_HEAD_DIM, k_cache, v_cache, pages + s * seq_pages, pos0 + s, q_heads,
+                     kv_heads, max_ctx, eps);
 }
 
 // The RoPE table of the fused decode attention: cs[2 (p 64 + i)] = cos and cs[2 (p 64 + i) + 1] =
