@@ -111,7 +111,7 @@ x0ne_status x0ne_gpu_launch_3d(x0ne_gpu* g, const char* name, uint32_t gx, uint3
    when a capture begins). The same shape runs the same kernels: the same bits. */
 x0ne_status x0ne_gpu_gemv(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n, uint64_t y,
                           int out_f32);
-/* The tiled matrix-core GEMM of x0ne_gpu_gemv past 64 rows with an explicit block tile (output
+/* The tiled matrix-core GEMM of x0ne_gpu_gemv past one row with an explicit block tile (output
    features x tokens; AUTO: the one x0ne_gpu_gemv picks) and operand layout, for kernel tests and
    tuning; no counterpart in the reference, whose Gpu::gemm is one cuBLAS call
    (gpu.rs:1098-1149). Y[n][rows] = X[n][cols] W^T, bf16 W and X, f32 accumulation in a fixed

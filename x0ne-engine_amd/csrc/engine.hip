@@ -555,8 +555,8 @@ x0ne_status plan(x0ne_engine* e) {
     // A second copy of the projections in 16-row panels (device.h), filled from the row-major
     // copy at load, for a batched engine (the few-row GEMM then reads one contiguous KiB of W per
     // step instead of 64 bytes of 16 rows) and for a prefill pass of more than one row (the
-    // tiled GEMM's loads fetch whole 1 KiB fragments: 25 TB/s from the L2 against 9.5
-    // row-major on MI355X). The prefill pass's GEMM inputs (normed rows, attention, SwiGLU) are
+    // tiled GEMM's loads fetch whole 1 KiB fragments; 2048 x 24576 x 4096 in bursts 334-343 us,
+    // row-major 344). The prefill pass's GEMM inputs (normed rows, attention, SwiGLU) are
     // then written in panels too. A batched engine's LM head has a panel copy as well.
     const bool dims16 = c.qkv_rows() % 16 == 0 && c.hidden % 16 == 0 && c.inter % 16 == 0;
     const uint64_t group = c.q_heads / c.kv_heads;
