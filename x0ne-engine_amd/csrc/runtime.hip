@@ -1103,8 +1103,9 @@ extern "C" x0ne_status x0ne_arena_scrub(x0ne_arena* a, uint64_t* zeroed) {
     if (!a) return fail(X0NE_ERR_ARENA, "null arena");
     if (!a->frozen) return fail(X0NE_ERR_ARENA, "the arena is not frozen");
     uint64_t total = 0;
+    x0ne_status st = X0NE_OK;
     const size_t n = a->regions.size();
-    for (size_t i = 0; i < n; ++i) {
+    for (size_t i = 0; i < n && st == X0NE_OK; ++i) {
         const auto& r = a->regions[i];
         if (r.cls != X0NE_CLASS_CLIENT_DATA) continue;
         total += r.len;
@@ -1120,12 +1121,17 @@ extern "C" x0ne_status x0ne_arena_scrub(x0ne_arena* a, uint64_t* zeroed) {
             end = a->regions[i + 1].offset + a->regions[i + 1].len;
         }
         a->gpu->counts.memsets++;
-        X0NE_HIP(hipMemsetAsync(a->base + r.offset, 0, end - r.offset, a->gpu->stream), "scrub");
+        const hipError_t e = hipMemsetAsync(a->base + r.offset, 0, end - r.offset, a->gpu->stream);
+        if (e != hipSuccess) st = gpu_fail(e, "scrub");
     }
+    // Also behind a refused fill: a request's copies from the caller's memory are queued on the
+    // stream without a wait, and its entry point returns after this.
     if (a->gpu) {
         a->gpu->counts.syncs++;
-        X0NE_HIP(hipStreamSynchronize(a->gpu->stream), "scrub");
+        const hipError_t e = hipStreamSynchronize(a->gpu->stream);
+        if (e != hipSuccess && st == X0NE_OK) st = gpu_fail(e, "scrub");
     }
+    if (st != X0NE_OK) return st;
     if (zeroed) *zeroed = total;
     return X0NE_OK;
 }
