@@ -413,6 +413,39 @@ def test_a_gpu_takes_its_slices_workspace_while_another_thread_captures(kernels)
     assert (got == kernels.gemm(w, rows, cols, x, n, True).view(np.uint32).ravel()).all()
 
 
+def test_a_gpu_takes_its_slices_workspace_at_the_first_call_with_slices(kernels):
+    """Refused calls, one row, and a shape whose tiles fill the chip leave a Gpu without the 64 MiB
+    workspace of the K slices; the first shape cut into slices takes it, once."""
+    from x0ne_core import Arena, Class, Error, Gpu
+    whole, cut = (6144, 1024, 60), (6148, 4096, 2)
+
+    def calls(gpu, a, sl):
+        def gemv(rows, cols, n):
+            gpu.gemv(a.ptr(sl["w"]), rows, cols, a.ptr(sl["x"]), n, a.ptr(sl["y"]), True)
+            gpu.sync()
+            return gpu.mem_info()[0]
+        free = [gpu.mem_info()[0]]
+        for bad in (lambda: gpu.gemv(a.ptr(sl["w"]), 0, 1024, a.ptr(sl["x"]), 60, a.ptr(sl["y"]), True),
+                    lambda: gpu.gemm_tiled(0, a.ptr(sl["w"]), 6, 1024, a.ptr(sl["x"]), 60, a.ptr(sl["y"]), True)):
+            with pytest.raises(Error):
+                bad()
+        free += [gpu.mem_info()[0], gemv(4096, 1024, 1), gemv(*whole), gemv(*cut), gemv(*cut)]
+        return [(free[0] - f) / (1 << 20) for f in free[1:]]
+
+    def measure():
+        gpu, a, sl = Gpu(), Arena(), {}
+        for name, size in (("w", 6148 * 4096 * 2), ("x", 60 * 4096 * 2), ("y", 60 * 6148 * 4)):
+            sl[name] = a.alloc(name, size, Class.CLIENT_DATA)
+        a.freeze(gpu)
+        a.scrub_client_data()
+        return calls(gpu, a, sl)
+
+    measure()  # the kernels' code is loaded
+    taken = measure()
+    print(f"MEASURE MiB taken after refused calls, one row, whole, cut, cut again: {taken}")
+    assert all(t < 32 for t in taken[:3]) and all(64 <= t < 96 for t in taken[3:]), taken
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_few_row_gemm_is_the_oracle_and_its_swiglu_the_swiglu_kernel(kernels, seed):
     """The batched step's projection kernel (2 to 64 rows of X, each W row read once) at every

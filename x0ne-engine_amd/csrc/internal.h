@@ -52,7 +52,7 @@ struct x0ne_gpu {
     // This device's copy of the library's static scratch array (runtime.hip, `scratch`), as
     // hipGetSymbolAddress gave it at x0ne_gpu_new with the device current.
     void* scratch = nullptr;
-    // K-slice sums of the tiled GEMM for calls on this Gpu (runtime.hip, tile_work), taken when
+    // K-slice sums of the tiled GEMM for calls on this Gpu (runtime.hip, own_parts), taken when
     // first needed and freed with the Gpu. Its calls run on one stream, one after the other.
     float* tile_parts = nullptr;
     bool tile_parts_refused = false;  // the allocation failed once: its calls stay unsplit
@@ -109,8 +109,10 @@ x0ne_status skinny(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols, con
 struct TileWork {
     float* parts = nullptr;
     uint64_t bytes = 0;
+    bool own = false;  // the Gpu's own, taken when the plan has slices
 };
 constexpr uint64_t TILE_PARTS_BYTES = 64ull << 20;  // room for every split that the plan prefers
+constexpr TileWork OWN_TILE_WORK = {nullptr, TILE_PARTS_BYTES, true};
 x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, uint64_t rows, uint64_t cols,
                        const void* x, uint64_t n, void* y, bool out_f32, TileWork work = {});
 // x0ne_gpu_gemv with the tiled GEMM's workspace given.

@@ -283,6 +283,25 @@ static constexpr uint64_t GEMM_MAX_BYTES = 0xFFFFFFF0ull;
 
 namespace x0ne {
 
+// The Gpu's own workspace for the tiled GEMM's slices, allocated at the first call whose plan has
+// slices or when a capture begins (a capture must not allocate); null without the memory for it: the
+// Gpu's GEMMs then stay unsplit.
+static float* own_parts(x0ne_gpu* g) {
+    if (!g->tile_parts && !g->tile_parts_refused && !g->capturing) {
+        // Another thread may have a capture of its own Gpu open: this thread's mode is relaxed for the
+        // allocation, so that it is neither refused nor ends that capture.
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+        if (hipMalloc((void**)&g->tile_parts, TILE_PARTS_BYTES) != hipSuccess) {
+            (void)hipGetLastError();
+            g->tile_parts = nullptr;
+            g->tile_parts_refused = true;
+        }
+        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    return g->tile_parts;
+}
+
 // ---- many rows: the tiled matrix-core GEMM of gemm.hip ----
 // The reference hands Gpu::gemm to cuBLAS (gpu.rs:1098-1149); past one row this library runs its
 // own tiled GEMM (x0ne_launch_gemm_tiles), the tile and the K slices chosen
@@ -301,8 +320,11 @@ x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, ui
                                          std::to_string(n) + " (rows a multiple of 4, of 16 with W in panels, "
                                          "cols of 8, W and X below 4 GiB, 16-byte aligned operands)");
     X0neTilePlan plan = {tile, 1};
-    if (tile == 0)
-        plan = x0ne_gemm_tile_plan((uint32_t)rows, (uint32_t)cols, (uint32_t)n, g->cus, work.parts ? work.bytes : 0);
+    if (tile == 0) {
+        auto pick = [&](uint64_t room) { return x0ne_gemm_tile_plan((uint32_t)rows, (uint32_t)cols, (uint32_t)n, g->cus, room); };
+        plan = pick(work.own || work.parts ? work.bytes : 0);
+        if (work.own && plan.slices > 1 && !(work.parts = own_parts(g))) plan = pick(0);
+    }
     const uint32_t flags = (out_f32 ? X0NE_TILE_F32 : 0u) | (wp ? X0NE_TILE_W_PANEL : 0u) | (xp ? X0NE_TILE_X_PANEL : 0u);
     g->counts.gemms++;
     g->counts.launches += plan.slices > 1 ? 2 : 1;
@@ -310,25 +332,6 @@ x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, ui
                                     g->stream),
              "tiled gemm");
     return X0NE_OK;
-}
-
-// The Gpu's own workspace for the tiled GEMM's slices, allocated at the first call that may use it
-// or when a capture begins (a capture must not allocate). Without the memory for it the Gpu's
-// GEMMs stay unsplit.
-static TileWork tile_work(x0ne_gpu* g) {
-    if (!g->tile_parts && !g->tile_parts_refused && !g->capturing) {
-        // Another thread may have a capture of its own Gpu open: this thread's mode is relaxed for the
-        // allocation, so that it is neither refused nor ends that capture.
-        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-        const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-        if (hipMalloc((void**)&g->tile_parts, TILE_PARTS_BYTES) != hipSuccess) {
-            (void)hipGetLastError();
-            g->tile_parts = nullptr;
-            g->tile_parts_refused = true;
-        }
-        if (relaxed) (void)hipThreadExchangeStreamCaptureMode(&mode);
-    }
-    return g->tile_parts ? TileWork{g->tile_parts, TILE_PARTS_BYTES} : TileWork{};
 }
 
 x0ne_status skinny(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols, const void* x, uint64_t n, void* y,
@@ -594,13 +597,13 @@ extern "C" x0ne_status x0ne_gpu_gemm_tiled(x0ne_gpu* g, uint32_t tile, uint32_t 
     if (!g) return fail(X0NE_ERR_GPU, "no device");
     if (tile > X0NE_GEMM_TILE_128x128) return fail(X0NE_ERR_FORMAT, "tiled gemm: tile " + std::to_string(tile));
     return x0ne::tiled_gemm(g, (int)tile, layout, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32 != 0,
-                            tile == X0NE_GEMM_TILE_AUTO ? tile_work(g) : TileWork{});
+                            tile == X0NE_GEMM_TILE_AUTO ? OWN_TILE_WORK : TileWork{});
 }
 
 extern "C" x0ne_status x0ne_gpu_gemv(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n,
                                      uint64_t y, int out_f32) {
     if (!g) return fail(X0NE_ERR_GPU, "no device");
-    return x0ne::gemv_rows(g, w, rows, cols, x, n, y, out_f32 != 0, n > 1 ? tile_work(g) : TileWork{});
+    return x0ne::gemv_rows(g, w, rows, cols, x, n, y, out_f32 != 0, OWN_TILE_WORK);
 }
 
 x0ne_status x0ne::gemv_rows(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n, uint64_t y,
@@ -919,7 +922,7 @@ extern "C" uint64_t x0ne_split_state_bytes(uint32_t q_heads, uint32_t splits) {
 extern "C" x0ne_status x0ne_gpu_capture_begin(x0ne_gpu* g) {
     if (!g) return fail(X0NE_ERR_GPU, "no device");
     if (g->capturing) return fail(X0NE_ERR_GPU, "a capture is already open");
-    (void)tile_work(g);
+    (void)own_parts(g);
     return x0ne::capture_begin(g);
 }
 
