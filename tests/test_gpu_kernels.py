@@ -979,6 +979,67 @@ def test_swiglu_of_every_gate_is_the_f64_value_rounded(kernels, seed):
     assert (same | ~ok).mean() > 0.99999  # numpy's exponential may differ in its last place
 
 
+def swiglu_fills(rng, rows, inter):
+    """Gate and up rows in which the f32 value settles none, some or all of a lane's eight."""
+    def n(*shape, scale=1.0):
+        return bf16_bits(O.bf16_round(rng.normal(0, scale, shape).astype(np.float32))).reshape(shape)
+    gate, up = n(rows, inter), n(rows, inter)
+    low = bf16_bits(O.bf16_round((-80.0 - np.abs(rng.normal(0, 20, (rows, inter)))).astype(np.float32))).reshape(rows, inter)
+    lane = np.arange(inter) % 8
+    odd = rng.integers(0, 1 << 16, (rows, inter)).astype(np.uint16)
+    return {"normal": (gate, up), "zero ups": (gate, up * 0), "half zero": (gate, np.where(rng.random((rows, inter)) < 0.5, 0, up)),
+            "zero gates": (np.where(rng.random((rows, inter)) < 0.9, np.uint16(0x8000), gate), odd),
+            "tiny": (n(rows, inter, scale=1e-20), n(rows, inter, scale=1e-20)), "low": (low, up),
+            "first low": (np.where(lane == 0, low, odd), up), "odd": (odd, rng.permutation(odd.ravel()).reshape(odd.shape)),
+            **{f"{k} low": (np.where(lane >= 8 - k, low, gate), up) for k in (1, 2, 3)},
+            "one lane's": (np.where(np.arange(inter) % 512 < 24, low, gate), up), "large": (gate & 0x7FFF | 0x4300, odd)}
+
+
+@pytest.mark.parametrize("rows,inter", [(1, 8), (8, 520), (11, 2056)])
+def test_swiglu_of_any_fill_is_the_f64_value_rounded(kernels, rows, inter):
+    """Lanes and wavefronts in which none, one, two, more or all of the values need f64, at ends inside a
+    wavefront and an 8-row group: the bits of single values, in rows and in panels."""
+    rng = np.random.default_rng(rows + inter)
+    for what, (gate, up) in swiglu_fills(rng, rows, inter).items():
+        gu = np.stack([gate, up], 1).astype(np.uint16)
+        fast = kernels.swiglu_rows(gu.ravel(), rows).reshape(rows, inter)
+        padded = np.concatenate([gu, np.zeros((rows, 2, 1), np.uint16)], -1)
+        single = kernels.swiglu_rows(padded.ravel(), rows).reshape(rows, inter + 1)[:, :-1]
+        assert (fast == single).all(), f"{what}: {(fast != single).sum()} of {fast.size} differ"
+        assert (kernels.swiglu_rows(gu.ravel(), rows, panel=True).reshape(rows, inter) == single).all(), what
+
+
+def test_swiglu_of_zeros_takes_no_longer(kernels):
+    """Rows of zero or tiny values take the time of others (2.1 to 2.5 times it where each such value is
+    computed in f64 by itself)."""
+    import time
+
+    from x0ne_core import Arena, Arg, Class
+    rows, inter = 2048, 12288
+    rng = np.random.default_rng(1)
+    g, a = kernels.gpu, Arena()
+    gs, os_ = a.alloc("gu", rows * 2 * inter * 2, Class.CLIENT_DATA), a.alloc("out", rows * inter * 2, Class.CLIENT_DATA)
+    a.freeze(g)
+    block = {k: np.concatenate(v, 1) for k, v in swiglu_fills(rng, 64, inter).items() if k in ("normal", "zero ups", "half zero", "tiny")}
+    us = {}
+    for what, gu in block.items():
+        a.write(gs, 0, np.tile(gu.astype(np.uint16), (rows // 64, 1)))
+        for kernel in ("x0ne_swiglu_bf16", "x0ne_swiglu_panel_bf16"):
+            args = [Arg.ptr(a.ptr(gs)), Arg.ptr(a.ptr(os_)), Arg.u32(inter)]
+            graph = g.capture(lambda: [g.launch(kernel, (inter // 2048, rows), 256, args) for _ in range(50)])
+            best = 1e9
+            for _ in range(6):
+                g.sync()
+                t = time.perf_counter()
+                g.launch_graph(graph)
+                g.sync()
+                best = min(best, time.perf_counter() - t)
+            us[what, kernel] = best / 50 * 1e6
+    print(f"MEASURE swiglu of {rows} x {2 * inter}, us: { {k: round(v, 1) for k, v in us.items()} }")
+    for (what, kernel), t in us.items():
+        assert t < 1.6 * us["normal", kernel], (what, kernel, us)
+
+
 @pytest.mark.parametrize("seed", range(20))
 def test_swiglu_is_the_oracle(kernels, seed):
     rng = O.Rng(600 + seed)

@@ -401,34 +401,53 @@ __device__ __forceinline__ bf16_t swiglu1(bf16_t g16, bf16_t u16) {
     const double g = (double)bf2f(g16), u = (double)bf2f(u16);
     return f2bf((float)(g / (1.0 + exp(-g)) * u));
 }
-// The f32 value's bf16, and whether it is surely swiglu1's. For |g| < 64, x = -g log2(e) is one
+// The f32 value's bf16, and whether it is surely swiglu1's. For -80 < g < 0, x = -g log2(e) is one
 // rounding of its exact sum (g's 8 bits times 15 of the constant's, and the rest), so e^-g is off by
 // |g| 2^-24 of itself plus the exponential's ulp; with the sum, the reciprocal (1 ulp) and the two
 // products the value is off by less than 2^-21 + |g| 2^-24, that is by 8 + |g| units of its last
-// place. Twice that is kept from the middle between two bf16 values (the low half word at 0x8000);
-// rounding is monotonic, so the f64 value lands on the same one. Zeros, the far ends of the exponents,
+// place; for g >= 0, where g e^-g < 1 holds the first part down, by 9. Twice that is kept from the
+// middle between two bf16 values (the low half word at 0x8000); rounding is monotonic, so the f64
+// value lands on the same one. Denormal values and zeros too: the reciprocal is normal, g times it is
+// below 2^-126 only for a g so small that the reciprocal is 1/2 (no rounding), and the last product's
+// rounding is half a unit; a zero keeps the product's sign. g <= -80, values from 2^101 on,
 // infinities and NaN are not sure.
 __device__ __forceinline__ bf16_t swiglu_f32(bf16_t g16, bf16_t u16, bool& sure) {
-    const float g = bf2f(g16), u = bf2f(u16), a = fabsf(g);
+    const float g = bf2f(g16), u = bf2f(u16);
     const float e = __builtin_amdgcn_exp2f(fmaf(-g, 7.0526076e-06f, -g * 1.44268798828125f));
     const float v = g * __builtin_amdgcn_rcpf(1.0f + e) * u;
     const uint32_t b = __float_as_uint(v), mag = b & 0x7FFFFFFFu;
     const int off = abs((int)(b & 0xFFFFu) - 0x8000);
-    sure = a < 64.0f && mag > 0x0D800000u && mag < 0x72000000u && off > 18 + (int)(2.0f * a);  // 2^-100 .. 2^101
+    sure = g > -80.0f && mag < 0x72000000u && off > (int)fmaxf(fmaf(-2.0f, g, 18.0f), 20.0f);
     return f2bf(v);
 }
-// Eight values from 16-byte aligned gate and up into 16 bytes at o, the first one's place; those that
-// are not sure are stored a second time.
+// Eight values from 16-byte aligned gate and up into 16 bytes at o, the first one's place. A stray
+// unsure value is computed again by itself and stored a second time; where a lane of the wavefront has
+// more than two, all eight of each lane are, their f64 chains side by side; and a wavefront whose first
+// gates are all out of range does without the f32 values. 2048 rows of 24576, us, with f64 for every
+// value / each unsure one by itself, zeros among them / now: N(0, 1) 46 / 28 / 28, zero ups 46 / 71 /
+// 28, half of them zero 41 / 59 / 28, gates of 80 to 84 (many products end midway) 43 / 70 / 43, of
+// -85 to -89 40 / 64 / 41.
 __device__ __forceinline__ void swiglu8(const bf16_t* gate, const bf16_t* up, bf16_t* o) {
     const uint4 g = *reinterpret_cast<const uint4*>(gate), u = *reinterpret_cast<const uint4*>(up);
     const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w};
     uint32_t ow[4], again = 0;
+    bool all = __all((gw[0] & 0xFFFFu) >= 0xC2A0u);  // g <= -80
+    if (!all) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        bool lo, hi;
-        ow[j] = (uint32_t)swiglu_f32((bf16_t)(gw[j] & 0xFFFFu), (bf16_t)(uw[j] & 0xFFFFu), lo);
-        ow[j] |= (uint32_t)swiglu_f32((bf16_t)(gw[j] >> 16), (bf16_t)(uw[j] >> 16), hi) << 16;
-        again |= (lo ? 0u : 1u << (2 * j)) | (hi ? 0u : 2u << (2 * j));
+        for (int j = 0; j < 4; ++j) {
+            bool lo, hi;
+            ow[j] = (uint32_t)swiglu_f32((bf16_t)(gw[j] & 0xFFFFu), (bf16_t)(uw[j] & 0xFFFFu), lo);
+            ow[j] |= (uint32_t)swiglu_f32((bf16_t)(gw[j] >> 16), (bf16_t)(uw[j] >> 16), hi) << 16;
+            again |= (lo ? 0u : 1u << (2 * j)) | (hi ? 0u : 2u << (2 * j));
+        }
+        all = __any(__popc(again) > 2);
+    }
+    if (all) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            ow[j] = (uint32_t)swiglu1((bf16_t)(gw[j] & 0xFFFFu), (bf16_t)(uw[j] & 0xFFFFu)) |
+                    ((uint32_t)swiglu1((bf16_t)(gw[j] >> 16), (bf16_t)(uw[j] >> 16)) << 16);
+        again = 0;
     }
     *reinterpret_cast<uint4*>(o) = make_uint4(ow[0], ow[1], ow[2], ow[3]);
     for (; again; again &= again - 1) {
