@@ -157,3 +157,19 @@ def oracle_from_tensors(cfg: O.Config, tensors: dict) -> O.Model:
 def top_two(row):
     s = np.sort(np.asarray(row, np.float32))
     return float(s[-1]), float(s[-2])
+
+
+def run_cpp(tmp_path, source: str, stdin: str = "") -> str:
+    """Builds tests/cpp/<source> against the built library with the host compiler, runs it and returns
+    what it printed; its own definitions of HIP calls come before the runtime library's."""
+    import subprocess
+
+    from x0ne_core._lib import LIB_PATH
+    exe = os.path.join(tmp_path, "program")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I", os.path.join(ROOT, "x0ne-engine_amd", "csrc"), os.path.join(ROOT, "tests", "cpp", source),
+                    LIB_PATH, f"-Wl,-rpath,{os.path.dirname(LIB_PATH)}", "-rdynamic", "-Wl,--allow-shlib-undefined",
+                    "-o", exe], check=True, capture_output=True, text=True)
+    r = subprocess.run([exe], input=stdin, capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0, r.stderr
+    return r.stdout

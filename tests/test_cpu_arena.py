@@ -8,7 +8,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from common import O
+from common import O, run_cpp
 
 POISON = 0xA5
 ALIGN = 256
@@ -165,15 +165,4 @@ def test_an_arena_is_planned_then_frozen_once():
 
 def test_a_device_scrub_drains_its_stream_also_when_a_fill_is_refused(tmp_path):
     """tests/cpp/scrub_drain.cpp on the built library, with HIP's answers given on the host."""
-    import os
-    import subprocess
-
-    from common import ROOT
-    from x0ne_core._lib import LIB_PATH
-    exe = tmp_path / "scrub_drain"
-    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
-                    "-I", os.path.join(ROOT, "x0ne-engine_amd", "csrc"), os.path.join(ROOT, "tests", "cpp", "scrub_drain.cpp"),
-                    LIB_PATH, f"-Wl,-rpath,{os.path.dirname(LIB_PATH)}", "-rdynamic", "-Wl,--allow-shlib-undefined",
-                    "-o", str(exe)], check=True, capture_output=True, text=True)
-    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
-    assert r.returncode == 0, r.stderr
+    run_cpp(tmp_path, "scrub_drain.cpp")

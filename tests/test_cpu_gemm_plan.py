@@ -1,0 +1,30 @@
+"""The tiled GEMM's plan (block tile and K slices for a shape) on the CPU: the built library's own, at 256
+CUs."""
+import numpy as np
+
+from common import run_cpp
+
+ROOM = 64 << 20  # the slices' workspace of a Gpu
+# Block tiles of launch.h by number: features, tokens, threads.
+TILES = {1: (256, 256, 512), 2: (256, 128, 512), 3: (128, 128, 256), 4: (64, 64, 256), 5: (128, 32, 128), 6: (16, 16, 64)}
+
+
+def plans(tmp_path, shapes, room=ROOM):
+    out = run_cpp(tmp_path, "tile_plan.cpp", "".join(f"{r} {c} {n} {room}\n" for r, c, n in shapes))
+    return [tuple(int(v) for v in line.split()) for line in out.splitlines()]
+
+
+def test_a_planned_grid_is_one_that_hip_launches(tmp_path):
+    """Operands up to 4 GiB and outputs up to the card's memory: a grid of at most 2^32 - 1 threads, in
+    slices that K and the workspace hold."""
+    shapes = []
+    for cols in (8, 24, 64, 1024, 4096):
+        for lr in np.arange(2, 28.2, 0.5):
+            for ln in np.arange(1, 28.2, 0.5):
+                rows, n = int(2 ** lr) // 4 * 4, int(2 ** ln)
+                if rows >= 4 and rows * cols < 1 << 31 and n * cols < 1 << 31 and rows * n < 140 << 30:
+                    shapes.append((rows, cols, n))
+    for (rows, cols, n), (tile, slices) in zip(shapes, plans(tmp_path, shapes)):
+        bf, bt, threads = TILES[tile]
+        assert -(-rows // bf) * -(-n // bt) * slices * threads < 1 << 32, (rows, cols, n, tile, slices)
+        assert slices == 1 or (slices <= -(-cols // 64) and slices * n * rows * 4 <= ROOM), (rows, cols, n, tile, slices)

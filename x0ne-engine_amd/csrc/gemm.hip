@@ -989,6 +989,7 @@ X0neTilePlan x0ne_gemm_tile_plan(uint32_t rows, uint32_t cols, uint32_t n, uint3
         const uint64_t tiles = tile_count(k, rows, n), part = (uint64_t)n * rows * 4;
         const double stream = 2.0 + 2.0 * rows * cols / 9.3e6, reads = (double)tiles * stages * (k.bf + k.bt) * 128 / 21e6;
         for (uint32_t slices : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u}) {
+            if (tiles * slices * k.threads > UINT32_MAX) break;  // more than HIP launches
             // A slice holds at least 4 stages, and all slices' blocks come to a few per CU at most.
             if (slices > 1 && (slices > stages / 4 || slices * part > parts_bytes || tiles * slices > 24ull * cus)) break;
             const double per_cu = std::ceil((double)(tiles * slices) / cus);
