@@ -125,8 +125,14 @@ enum {
     X0NE_GEMM_TILE_AUTO = 0,
     X0NE_GEMM_TILE_256x256 = 1,
     X0NE_GEMM_TILE_256x128 = 2,
-    X0NE_GEMM_TILE_128x128 = 3
+    X0NE_GEMM_TILE_128x128 = 3,
+    X0NE_GEMM_TILE_64x64 = 4,
+    X0NE_GEMM_TILE_128x32 = 5,
+    X0NE_GEMM_TILE_16x16 = 6
 };
+/* Added to a named tile: K cut into s (2 .. 255) slices, at most one per 64 columns, whose f32 sums
+   (s n rows of them) fit the Gpu's workspace; a named tile alone sums K in one piece. */
+#define X0NE_GEMM_SLICES(s) ((uint32_t)(s) << 8)
 enum { X0NE_GEMM_W_PANELS = 1, X0NE_GEMM_X_PANELS = 2 };
 x0ne_status x0ne_gpu_gemm_tiled(x0ne_gpu* g, uint32_t tile, uint32_t layout, uint64_t w, uint64_t rows, uint64_t cols,
                                 uint64_t x, uint64_t n, uint64_t y, int out_f32);

@@ -28,3 +28,18 @@ def test_a_planned_grid_is_one_that_hip_launches(tmp_path):
         bf, bt, threads = TILES[tile]
         assert -(-rows // bf) * -(-n // bt) * slices * threads < 1 << 32, (rows, cols, n, tile, slices)
         assert slices == 1 or (slices <= -(-cols // 64) and slices * n * rows * 4 <= ROOM), (rows, cols, n, tile, slices)
+
+
+def test_the_gpu_tests_shapes_reach_every_tile_that_the_plan_uses(tmp_path):
+    """The tiles, in one piece and in slices, that the plan picks for the projections of the Qwen3 shapes by
+    2 to 2048 rows are among those it picks for the GEMM tests of test_gpu_kernels.py."""
+    from bench import QWEN3_0_6B, QWEN3_8B, QWEN3_32B
+    from test_gpu_kernels import PLANNED, PREFILL, PREFILL_N
+    shapes = []
+    for m in (QWEN3_0_6B, QWEN3_8B, QWEN3_32B):
+        h, i, d = m["hidden_size"], m["intermediate_size"], m["head_dim"]
+        q, kv = m["num_attention_heads"] * d, m["num_key_value_heads"] * d
+        shapes += [(r, c, n) for r, c in ((q + 2 * kv, h), (h, q), (2 * i, h), (h, i)) for n in range(2, 2049)]
+    used = {(t, s > 1) for t, s in plans(tmp_path, shapes)}
+    tested = {(t, s > 1) for t, s in plans(tmp_path, PLANNED + [(r, c, PREFILL_N) for _, r, c in PREFILL])}
+    assert used <= tested, used - tested

@@ -230,9 +230,9 @@ def test_gemv_is_the_oracle_on_random_shapes(kernels, seed):
 
 @pytest.mark.parametrize("seed", range(16))
 def test_gemm_is_the_oracle_gemv_of_every_row(kernels, seed):
-    """Gpu::gemm over many rows (the few-row matrix-core kernel up to 64 rows, this library's
-    tiled matrix-core GEMM past them when W's rows are a multiple of 4, a GEMV per row of X
-    otherwise): every row of Y is the oracle's GEMV of that row of X within the GEMV tolerance
+    """Gpu::gemm over many rows (this library's tiled matrix-core GEMM when W's rows are a multiple of
+    4, else and for a few rows of a small W the few-row matrix-core kernel up to 64 rows, a GEMV per
+    row of X past them): every row of Y is the oracle's GEMV of that row of X within the GEMV tolerance
     (gpu_kernels.rs:331-393), at tile edges of both sides and K tails. The bf16 output is the f32
     output rounded where the same kernel serves both (one accumulation, two stores); the per-row
     GEMV may differ between the two, and, as the reference does for its GEMV
@@ -262,7 +262,7 @@ def test_gemm_is_the_oracle_gemv_of_every_row(kernels, seed):
     assert (kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, True).view(np.uint32) == f.view(np.uint32)).all(), what
 
 
-TILES = {"256x256": 1, "256x128": 2, "128x128": 3}
+TILES = {"256x256": 1, "256x128": 2, "128x128": 3, "64x64": 4, "128x32": 5, "16x16": 6}
 W_PANELS, X_PANELS = 1, 2
 
 
@@ -303,8 +303,38 @@ def test_the_tiled_gemm_is_the_oracle_gemv_at_every_tile(kernels, tile, seed):
         assert (pb == b).all(), f"{what}: layout {layout} bf16"
 
 
-@pytest.mark.parametrize("name,rows,cols", [("qkv", 6144, 4096), ("o", 4096, 4096), ("gate_up", 24576, 4096),
-                                            ("down", 4096, 12288)])
+@pytest.mark.parametrize("tile", sorted(TILES))
+@pytest.mark.parametrize("n,rows,cols,slices", [(1, 16, 128, 2), (17, 132, 72, 2), (33, 272, 1000, 16), (65, 60, 1032, 3),
+                                                (130, 528, 776, 12), (257, 260, 520, 4)])
+def test_the_tiled_gemm_in_slices_at_every_tile(kernels, tile, n, rows, cols, slices):
+    """Each block tile with K cut into a named number of slices, up to one per 64-column stage, at ends
+    inside a tile, a stage and a slice: each output within f32 sums of the exact product, the bf16
+    output the f32 output rounded, the same bits on a second call and from panels. Counts that K or
+    the workspace does not hold are refused, as are a single slice and slices of no named tile."""
+    from x0ne_core import FormatError
+    rng = O.Rng(3000 + n + TILES[tile])
+    w, x = bf16s_with_edges(rng, rows * cols, 1e-2), bf16s_with_edges(rng, n * cols, 1.0)
+    t = TILES[tile] | slices << 8
+
+    def gemm(out_f32, layout=0, t=t):
+        return kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, out_f32, tile=t, layout=layout)
+    f, b = gemm(True), gemm(False)
+    W, X = w.reshape(rows, cols).astype(np.float64), x.reshape(n, cols).astype(np.float64)
+    r = np.abs(f.astype(np.float64) - X @ W.T) / (1e-5 * (np.abs(X) @ np.abs(W).T) + 1e-30)
+    assert (r <= 1.0).all(), f"worst ratio {r.max():.3f}"
+    assert (b == bf16_bits(f).reshape(b.shape)).all()
+    for layout in [0, X_PANELS] + ([W_PANELS, W_PANELS | X_PANELS] if rows % 16 == 0 else []):
+        assert (gemm(True, layout).view(np.uint32) == f.view(np.uint32)).all(), f"layout {layout}"
+    for bad in (TILES[tile] | 1 << 8, TILES[tile] | (-(-cols // 64) + 1) << 8, TILES[tile] | 256 << 8, 2 << 8, 7):
+        with pytest.raises(FormatError):
+            gemm(True, t=bad)
+
+
+PREFILL = [("qkv", 6144, 4096), ("o", 4096, 4096), ("gate_up", 24576, 4096), ("down", 4096, 12288)]
+PREFILL_N = 300
+
+
+@pytest.mark.parametrize("name,rows,cols", PREFILL)
 def test_the_tiled_gemm_at_the_prefill_shapes(kernels, name, rows, cols):
     """Qwen3-8B's four projections as a 2048-row prefill pass runs them, the tile the library
     picks for each (x0ne_gpu_gemv past 64 rows), on 300 tokens (two token tiles of every
@@ -312,7 +342,7 @@ def test_the_tiled_gemm_at_the_prefill_shapes(kernels, name, rows, cols):
     (the oracle's GEMV arithmetic) within the GEMV tolerance; the engine's form (W and X in
     panels, the same tile) gives the same bits."""
     rng = np.random.default_rng(rows + cols)
-    n = 300
+    n = PREFILL_N
     w = O.bf16_round(rng.normal(0, 0.02, rows * cols).astype(np.float32))
     x = O.bf16_round(rng.normal(0, 1.0, n * cols).astype(np.float32))
     f = kernels.gemm(bf16_bits(w), rows, cols, bf16_bits(x), n, True)
@@ -327,10 +357,14 @@ def test_the_tiled_gemm_at_the_prefill_shapes(kernels, name, rows, cols):
     assert (p.view(np.uint32) == f.view(np.uint32)).all(), f"{name}: panels"
 
 
-@pytest.mark.parametrize("rows,cols,n", [(64, 4096, 65), (1000, 2056, 65), (260, 12288, 100), (516, 4104, 200),
-                                         (4096, 4096, 257), (1024, 3072, 777), (2052, 1032, 333), (4, 1024, 65),
-                                         (4, 2056, 17), (132, 12296, 9), (6148, 4096, 2), (4096, 4096, 9), (4096, 4096, 31),
-                                         (24576, 1024, 64)])
+# rows, cols, n: with the shapes above every tile that the plan uses, in one piece and in slices
+# (test_cpu_gemm_plan.py).
+PLANNED = [(64, 4096, 65), (1000, 2056, 65), (260, 12288, 100), (516, 4104, 200), (4096, 4096, 257), (1024, 3072, 777),
+           (2052, 1032, 333), (4, 1024, 65), (4, 2056, 17), (132, 12296, 9), (6148, 4096, 2), (4096, 4096, 9),
+           (4096, 4096, 31), (24576, 1024, 64), (20480, 3080, 17), (10244, 5128, 18), (24576, 2056, 31), (4096, 1032, 1025), (8196, 2056, 32)]
+
+
+@pytest.mark.parametrize("rows,cols,n", PLANNED)
 def test_the_gemm_of_few_tiles_cuts_k_into_slices(kernels, rows, cols, n):
     """Gpu::gemm past a row where the tiles are too few for the chip: the K slices and their
     reduction, and the small tiles, at ends inside a tile, a stage and a slice. Against float64 products within the

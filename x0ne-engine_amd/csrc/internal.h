@@ -105,7 +105,7 @@ x0ne_status skinny(x0ne_gpu* g, const void* w, uint64_t rows, uint64_t cols, con
 // layout X0NE_GEMM_W_PANELS | X0NE_GEMM_X_PANELS names the operands held in 16-row panels.
 // With tile 0 a shape of few tiles cuts K into slices when `work` has room for their sums (the
 // same shape and room: the same kernels, the same bits); launches sharing it must not overlap.
-// Without, an output's bits do not depend on n.
+// Without, an output's bits do not depend on n. slices > 1: that many with a named tile, in `work`.
 struct TileWork {
     float* parts = nullptr;
     uint64_t bytes = 0;
@@ -114,7 +114,7 @@ struct TileWork {
 constexpr uint64_t TILE_PARTS_BYTES = 64ull << 20;  // room for every split that the plan prefers
 constexpr TileWork OWN_TILE_WORK = {nullptr, TILE_PARTS_BYTES, true};
 x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, uint64_t rows, uint64_t cols,
-                       const void* x, uint64_t n, void* y, bool out_f32, TileWork work = {});
+                       const void* x, uint64_t n, void* y, bool out_f32, TileWork work = {}, uint32_t slices = 1);
 // x0ne_gpu_gemv with the tiled GEMM's workspace given.
 x0ne_status gemv_rows(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n, uint64_t y,
                       bool out_f32, TileWork work);

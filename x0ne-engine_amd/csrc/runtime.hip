@@ -309,7 +309,7 @@ static float* own_parts(x0ne_gpu* g) {
 // same kernels, and each output is summed in a fixed order: results are the same from call to
 // call.
 x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, uint64_t rows, uint64_t cols,
-                       const void* x, uint64_t n, void* y, bool out_f32, TileWork work) {
+                       const void* x, uint64_t n, void* y, bool out_f32, TileWork work, uint32_t slices) {
     const bool wp = layout & X0NE_GEMM_W_PANELS, xp = layout & X0NE_GEMM_X_PANELS;
     const uint64_t xrows = xp ? (n + 15) / 16 * 16 : n;
     if (rows == 0 || cols == 0 || n == 0 || rows % 4 != 0 || cols % 8 != 0 || (wp && rows % 16 != 0) ||
@@ -319,8 +319,13 @@ x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, ui
         return fail(X0NE_ERR_FORMAT, "tiled gemm: " + std::to_string(rows) + "x" + std::to_string(cols) + ", n " +
                                          std::to_string(n) + " (rows a multiple of 4, of 16 with W in panels, "
                                          "cols of 8, W and X below 4 GiB, 16-byte aligned operands)");
-    X0neTilePlan plan = {tile, 1};
-    if (tile == 0) {
+    X0neTilePlan plan = {tile, slices};
+    if (slices > 1) {
+        if (slices > (cols + 63) / 64 || n > work.bytes / (rows * 4 * slices))
+            return fail(X0NE_ERR_FORMAT, "tiled gemm: " + std::to_string(slices) + " slices of " + std::to_string(rows) +
+                                             "x" + std::to_string(cols) + ", n " + std::to_string(n));
+        if (!work.parts && !(work.own && (work.parts = own_parts(g)))) return fail(X0NE_ERR_GPU, "tiled gemm: no workspace for the slices");
+    } else if (tile == 0) {
         auto pick = [&](uint64_t room) { return x0ne_gemm_tile_plan((uint32_t)rows, (uint32_t)cols, (uint32_t)n, g->cus, room); };
         plan = pick(work.own || work.parts ? work.bytes : 0);
         if (work.own && plan.slices > 1 && !(work.parts = own_parts(g))) plan = pick(0);
@@ -595,9 +600,11 @@ extern "C" x0ne_status x0ne_gpu_gemv_fused(x0ne_gpu* g, const x0ne_gemv_fused* d
 extern "C" x0ne_status x0ne_gpu_gemm_tiled(x0ne_gpu* g, uint32_t tile, uint32_t layout, uint64_t w, uint64_t rows,
                                            uint64_t cols, uint64_t x, uint64_t n, uint64_t y, int out_f32) {
     if (!g) return fail(X0NE_ERR_GPU, "no device");
-    if (tile > X0NE_GEMM_TILE_128x128) return fail(X0NE_ERR_FORMAT, "tiled gemm: tile " + std::to_string(tile));
-    return x0ne::tiled_gemm(g, (int)tile, layout, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32 != 0,
-                            tile == X0NE_GEMM_TILE_AUTO ? OWN_TILE_WORK : TileWork{});
+    const uint32_t named = tile & 0xFF, slices = tile >> 8;
+    if (named > X0NE_GEMM_TILE_16x16 || slices > 255 || slices == 1 || (slices && named == X0NE_GEMM_TILE_AUTO))
+        return fail(X0NE_ERR_FORMAT, "tiled gemm: tile " + std::to_string(tile));
+    return x0ne::tiled_gemm(g, (int)named, layout, (const void*)w, rows, cols, (const void*)x, n, (void*)y, out_f32 != 0,
+                            OWN_TILE_WORK, slices ? slices : 1);
 }
 
 extern "C" x0ne_status x0ne_gpu_gemv(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t cols, uint64_t x, uint64_t n,

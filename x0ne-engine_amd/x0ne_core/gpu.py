@@ -172,8 +172,8 @@ class Gpu:
 
     def gemm_tiled(self, tile: int, w: int, rows: int, cols: int, x: int, n: int, y: int, out_f32: bool,
                    layout: int = 0):
-        """The tiled matrix-core GEMM with block tile `tile` (x0ne_gpu_gemm_tiled; 0 picks one),
-        layout bit 0 W in 16-row panels, bit 1 X in panels."""
+        """The tiled matrix-core GEMM with block tile `tile` (x0ne_gpu_gemm_tiled; 0 picks one; a
+        named tile | s << 8 cuts K into s slices), layout bit 0 W in 16-row panels, bit 1 X in panels."""
         check(lib().x0ne_gpu_gemm_tiled(self.h, tile, layout, w, rows, cols, x, n, y, int(out_f32)), "gemm_tiled")
 
     def gemv_fused(self, **fields) -> None:
