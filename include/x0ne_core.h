@@ -127,8 +127,7 @@ enum {
     X0NE_GEMM_TILE_256x128 = 2,
     X0NE_GEMM_TILE_128x128 = 3,
     X0NE_GEMM_TILE_64x64 = 4,
-    X0NE_GEMM_TILE_128x32 = 5,
-    X0NE_GEMM_TILE_16x16 = 6
+    X0NE_GEMM_TILE_16x16 = 5
 };
 /* Added to a named tile: K cut into s (2 .. 255) slices, at most one per 64 columns, whose f32 sums
    (s n rows of them) fit the Gpu's workspace; a named tile alone sums K in one piece. */

@@ -6,7 +6,7 @@ from common import run_cpp
 
 ROOM = 64 << 20  # the slices' workspace of a Gpu
 # Block tiles of launch.h by number: features, tokens, threads.
-TILES = {1: (256, 256, 512), 2: (256, 128, 512), 3: (128, 128, 256), 4: (64, 64, 256), 5: (128, 32, 128), 6: (16, 16, 64)}
+TILES = {1: (256, 256, 512), 2: (256, 128, 512), 3: (128, 128, 256), 4: (64, 64, 256), 5: (16, 16, 64)}
 
 
 def plans(tmp_path, shapes, room=ROOM):

@@ -901,18 +901,17 @@ __device__ __forceinline__ void gemm_tiles(const bf16_t* __restrict__ w, const b
             return;                                                                                                   \
         gemm_tiles<WF, WT, NWF, NWT, STAGES>(w, x, y, rows, cols, n, flags, slices, parts, lds);                      \
     }
-// Block tiles from sweeps on MI355X over the Qwen3 projections at 2 to 2048 rows of X: 256 x 256
-// of 8 wavefronts (64 features x 128 tokens each; two per SIMD; four stages of 32 columns in
-// their place: 5-7 % slower row-major, level in panels), 256 x 128 of 8 (64 x 64 each), 64 x 64 of 4
-// (32 x 32 each, two blocks per CU), 128 x 32 of 2 (64 x 32 each, two blocks), 16 x 16 of one (ten
-// blocks), and 128 x 128 of 4, which a caller may name but no shape is best on. The small tiles
+// Block tiles from sweeps on MI355X: 256 x 256 of 8 wavefronts (64 features x 128 tokens each; two per
+// SIMD; four stages of 32 columns in their place: 5-7 % slower row-major, level in panels), 256 x 128
+// of 8 and 128 x 128 of 4 (64 x 64 each), 64 x 64 of 4 (32 x 32 each, two blocks per CU) and 16 x 16 of
+// one (ten blocks). 128 x 32 of two wavefronts was best for none of the Qwen3 projections but 10240 x
+// 5120 by 17 to 32 (26 us, 64 x 64 28), and far off the best on 16384 columns. The small tiles
 // stream W at 4-6 TB/s where the few-row kernels above, which read 64 bytes of 16 rows per load,
-// reach 1-4 on row-major W: 16 x 51200 x 5120 149 -> 97 us, 64 x 24576 x 4096 130 -> 47.
+// reach 1-4 on row-major W: 16 x 51200 x 5120 147 -> 106 us, 64 x 24576 x 4096 129 -> 47.
 X0NE_TILES(x0ne_gemm_tiles_256x256_bf16, 64, 128, 4, 2, 2)
 X0NE_TILES(x0ne_gemm_tiles_256x128_bf16, 64, 64, 4, 2, 3)
 X0NE_TILES(x0ne_gemm_tiles_128x128_bf16, 64, 64, 2, 2, 4)
 X0NE_TILES(x0ne_gemm_tiles_64x64_bf16, 32, 32, 2, 2, 4)
-X0NE_TILES(x0ne_gemm_tiles_128x32_bf16, 64, 32, 2, 1, 3)
 X0NE_TILES(x0ne_gemm_tiles_16x16_bf16, 16, 16, 1, 1, 4)
 
 // x0ne_gemm_tiles_reduce: y[t][f] = the f32 (flags TILE_F32) or bf16 of the sum over slices, in
@@ -948,20 +947,21 @@ struct TileKind {
     const void* fn;
     uint32_t bf, bt;  // block tile: features x tokens
     uint32_t threads;
-    // The plan's estimate, us on MI355X: a block's start and end, one stage of a block alone on
-    // its CU, and one stage of each block where several share a CU (0: they take turns).
+    // The plan's estimate, us on MI355X: a round of blocks' start and end (a CU holds `resident` blocks at
+    // once), one stage of a block alone on its CU, and one stage of each block where several share a
+    // CU (0: they take turns).
+    uint32_t resident;
     double fixed, stage, shared;
 };
 
 TileKind tile_kind(int tile) {
     switch (tile) {
-        case X0NE_TILE_256x256: return {(const void*)&x0ne_gemm_tiles_256x256_bf16, 256, 256, 512, 11.0, 1.2, 0};
-        case X0NE_TILE_256x128: return {(const void*)&x0ne_gemm_tiles_256x128_bf16, 256, 128, 512, 3.9, 0.98, 0};
-        case X0NE_TILE_128x128: return {(const void*)&x0ne_gemm_tiles_128x128_bf16, 128, 128, 256, 0, 0, 0};
-        case X0NE_TILE_64x64: return {(const void*)&x0ne_gemm_tiles_64x64_bf16, 64, 64, 256, 1.9, 0.17, 0.25};
-        case X0NE_TILE_128x32: return {(const void*)&x0ne_gemm_tiles_128x32_bf16, 128, 32, 128, 5.3, 0.38, 0.39};
-        case X0NE_TILE_16x16: return {(const void*)&x0ne_gemm_tiles_16x16_bf16, 16, 16, 64, 1.9, 0.14, 0.037};
-        default: return {nullptr, 0, 0, 0, 0, 0, 0};
+        case X0NE_TILE_256x256: return {(const void*)&x0ne_gemm_tiles_256x256_bf16, 256, 256, 512, 1, 8.1, 1.52, 0};
+        case X0NE_TILE_256x128: return {(const void*)&x0ne_gemm_tiles_256x128_bf16, 256, 128, 512, 1, 4.0, 0.96, 0};
+        case X0NE_TILE_128x128: return {(const void*)&x0ne_gemm_tiles_128x128_bf16, 128, 128, 256, 1, 2.5, 0.83, 0};
+        case X0NE_TILE_64x64: return {(const void*)&x0ne_gemm_tiles_64x64_bf16, 64, 64, 256, 2, 1.4, 0.26, 0.25};
+        case X0NE_TILE_16x16: return {(const void*)&x0ne_gemm_tiles_16x16_bf16, 16, 16, 64, 10, 0.75, 0.155, 0.038};
+        default: return {nullptr, 0, 0, 0, 1, 0, 0, 0};
     }
 }
 
@@ -972,32 +972,37 @@ uint64_t tile_count(const TileKind& k, uint32_t rows, uint32_t n) {
 }  // namespace
 
 // The tile and the K slices for a shape: the pair that an estimate of the time puts first. The
-// estimate is a block's fixed and per-stage time over the blocks of the fullest CU, not less than
-// W's stream (9.3 TB/s and 2 us) or the tiles' reads from the L2 (21 TB/s), and for several slices
-// the reduction (1 us and the parts at 2.2 TB/s). The constants are fitted to a sweep on MI355X of
-// the 12 Qwen3-0.6B, -8B and -32B projections at 27 counts from 2 to 2048 rows, row-major and in
-// panels, weights rotating: the picked pair takes 1.2 % longer than the best one on average, 18 %
-// at worst (777 x 4096 x 12288: 256 x 256 in 4 slices, 92 us; unsplit 256 x 128 159, 256 x 256 251;
-// 8 x 4096 x 12288: 16 x 16 in 4 slices, 22 us; 64 x 64 in 4 slices 25).
+// estimate is a block's time per round and per stage over the blocks of the fullest CU, not less than
+// W's stream (9.5 TB/s and 2 us) or the tiles' reads from the L2 (19.5 TB/s); 1.065 times it where
+// all slices start on the same memory channels (rows and slices of whole 4 KiB: 4096 x 8192 by 2 in
+// 3 slices 18.0 us, in 4 20.4; 4096 x 12288 by 17 in 3 28.3, in 4 23.8); and for several slices
+// the reduction (1 us and the parts at 2.3 TB/s). The constants are fitted to sweeps on MI355X of the
+// 12 Qwen3-0.6B, -8B and -32B projections by 2 to 2048 rows, row-major and in panels, and of a grid
+// of 4 to 65536 x 8 to 16384 by 2 to 1000, weights rotating: over the projections the picked pair takes
+// 1.0 % longer than the best one on average and 18 % at worst, over the grid 2.0 and 30 % (a round's
+// blocks without their start and end, no 128 x 128, and 128 x 32: 1.9 and 20 %, 4.0 and 93 %: 65536 x
+// 128 by 512 57 us in 64 x 64 tiles, 31 in 256 x 256).
 X0neTilePlan x0ne_gemm_tile_plan(uint32_t rows, uint32_t cols, uint32_t n, uint32_t cus, uint64_t parts_bytes) {
     const uint32_t stages = (cols + 63) / 64;
     X0neTilePlan best = {X0NE_TILE_256x256, 1};
     double best_us = 1e30;
     auto four = [](double a) { return a * a * a * a; };
-    for (int tile : {X0NE_TILE_16x16, X0NE_TILE_128x32, X0NE_TILE_64x64, X0NE_TILE_256x128, X0NE_TILE_256x256}) {
+    for (int tile : {X0NE_TILE_16x16, X0NE_TILE_64x64, X0NE_TILE_128x128, X0NE_TILE_256x128, X0NE_TILE_256x256}) {
         const TileKind k = tile_kind(tile);
         const uint64_t tiles = tile_count(k, rows, n), part = (uint64_t)n * rows * 4;
-        const double stream = 2.0 + 2.0 * rows * cols / 9.3e6, reads = (double)tiles * stages * (k.bf + k.bt) * 128 / 21e6;
+        const double stream = 2.0 + 2.0 * rows * cols / 9.5e6, reads = (double)tiles * stages * (k.bf + k.bt) * 128 / 19.5e6;
         for (uint32_t slices : {1u, 2u, 3u, 4u, 6u, 8u, 12u, 16u}) {
             if (tiles * slices * k.threads > UINT32_MAX) break;  // more than HIP launches
             // A slice holds at least 4 stages, and all slices' blocks come to a few per CU at most.
             if (slices > 1 && (slices > stages / 4 || slices * part > parts_bytes || tiles * slices > 24ull * cus)) break;
-            const double per_cu = std::ceil((double)(tiles * slices) / cus);
+            const double per_cu = std::ceil((double)(tiles * slices) / cus), rounds = std::ceil(per_cu / k.resident);
             const double steps = std::ceil((double)stages / slices);
-            double us = k.shared > 0 ? k.fixed + steps * std::max(per_cu * k.shared, k.stage)
-                                     : per_cu * (k.fixed + steps * k.stage);
+            double us = rounds * k.fixed + steps * (k.shared > 0 ? std::max(per_cu * k.shared, k.stage) : per_cu * k.stage);
             us = std::sqrt(std::sqrt(four(us) + four(stream) + four(reads)));
-            if (slices > 1) us += 1.0 + (double)slices * part / 2.2e6;
+            if (slices > 1) {
+                if (cols % 2048 == 0 && stages % slices == 0 && stages / slices % 32 == 0) us *= 1.065;
+                us += 1.0 + (double)slices * part / 2.3e6;
+            }
             if (us < best_us) best_us = us, best = {tile, slices};
         }
     }

@@ -111,7 +111,9 @@ struct TileWork {
     uint64_t bytes = 0;
     bool own = false;  // the Gpu's own, taken when the plan has slices
 };
-constexpr uint64_t TILE_PARTS_BYTES = 64ull << 20;  // room for every split that the plan prefers
+// Room for every split that the plan prefers for the Qwen3 projections, but the 32B shape's O and down
+// past 1536 rows, which would take 94 to 126 MB and go unsplit or in fewer slices.
+constexpr uint64_t TILE_PARTS_BYTES = 64ull << 20;
 constexpr TileWork OWN_TILE_WORK = {nullptr, TILE_PARTS_BYTES, true};
 x0ne_status tiled_gemm(x0ne_gpu* g, int tile, uint32_t layout, const void* w, uint64_t rows, uint64_t cols,
                        const void* x, uint64_t n, void* y, bool out_f32, TileWork work = {}, uint32_t slices = 1);

@@ -56,8 +56,7 @@ enum {
     X0NE_TILE_256x128 = 2,
     X0NE_TILE_128x128 = 3,
     X0NE_TILE_64x64 = 4,
-    X0NE_TILE_128x32 = 5,
-    X0NE_TILE_16x16 = 6
+    X0NE_TILE_16x16 = 5
 };
 enum { X0NE_TILE_F32 = 1, X0NE_TILE_W_PANEL = 2, X0NE_TILE_X_PANEL = 4 };
 struct X0neTilePlan {

@@ -623,9 +623,11 @@ x0ne_status x0ne::gemv_rows(x0ne_gpu* g, uint64_t w, uint64_t rows, uint64_t col
     // few-row kernel, whose wavefronts split K with all their loads in flight, is the faster one, for
     // as many rows as its steps are few (us, few-row against tiled: 4096 x 1024 by 8 rows 5.5 / 6.6,
     // by 32 6.7 / 6.9, by 48 8.4 / 7.0; 6144 x 1024, two blocks on some CUs, by 16 6.5 / 6.7, by 24
-    // 7.4 / 6.9; 4096 x 4096 by 4 10.6 / 11.2, by 16 12.8 / 11.5). From 50 MB of W on the tiled GEMM at
-    // every count: 6144 x 4096 by 2 15.4 / 14.0.
-    const uint64_t few = cols > 2048 ? 8 : cols > 1024 || rows > 16ull * g->cus ? 16 : 32;
+    // 7.4 / 6.9; 4096 x 4096 by 4 10.6 / 11.2, by 16 12.8 / 11.5; of less than a group of 16 rows, 4 x
+    // 4096 by 9 7.0 / 8.2, by 17 9.3 / 8.2). From 40 MB of W on the tiled GEMM at every count: level at
+    // first (4096 x 5120 by 2 12.3 / 13.3, by 8 14.5 / 13.1; 6144 x 4096 by 2 15.7 / 14.0), then the
+    // faster one (10240 x 5120 by 2 30.8 / 23.1).
+    const uint64_t few = cols > 4096 || (cols > 2048 && rows >= 16) ? 8 : cols > 1024 || rows > 16ull * g->cus ? 16 : 32;
     const bool small = 2 * rows * cols < 40'000'000 && n <= few;
     if (n >= 2 && !small && cols % 8 == 0 && rows % 4 == 0 && n <= UINT32_MAX && rows * cols * 2 <= GEMM_MAX_BYTES &&
         n * cols * 2 <= GEMM_MAX_BYTES && w % 16 == 0 && x % 16 == 0 && y % 16 == 0)

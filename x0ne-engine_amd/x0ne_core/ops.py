@@ -270,15 +270,16 @@ class Kernels:
         return a.read_array(ys, 0, rows, np.float32 if out_f32 else np.uint16)
 
     # x0ne_gpu_gemm_tiled's block tiles (features x tokens) and operand layouts
-    TILE_AUTO, TILE_256x256, TILE_256x128, TILE_128x128, TILE_64x64, TILE_128x32, TILE_16x16 = 0, 1, 2, 3, 4, 5, 6
+    TILE_AUTO, TILE_256x256, TILE_256x128, TILE_128x128, TILE_64x64, TILE_16x16 = 0, 1, 2, 3, 4, 5
     W_PANELS, X_PANELS = 1, 2
 
     def gemm(self, w, rows, cols, x, n, out_f32, tile=None, layout=0) -> np.ndarray:
         """Gpu::gemm over n rows of X (gpu.rs:1098-1149): Y[n][rows] = X[n][cols] W^T, the
         tiled matrix-core GEMM past one row (a few rows of a small W, and up to 64 where W's rows are
         no multiple of 4: the few-row kernel); tile names a block tile of the tiled GEMM
-        (x0ne_gpu_gemm_tiled; | s << 8: in s slices of K) at any row count, and layout asks it to read W and/or X in 16-row panels (uploaded as such from the row-major
-        arguments); returns Y (f32, or bf16 bits)."""
+        (x0ne_gpu_gemm_tiled; | s << 8: in s slices of K) at any row count, and layout asks it to read
+        W and/or X in 16-row panels (uploaded as such from the row-major arguments); returns Y (f32,
+        or bf16 bits)."""
         if rows == 0 or cols == 0 or n == 0 or w.size != rows * cols or x.size != n * cols:
             raise FormatError(f"gemm: W {w.size} for {rows}x{cols}, X {x.size} for {n} rows")
         if layout and tile is None:
