@@ -451,11 +451,14 @@ struct ExactPlan {
 // first: the wavefronts on the fullest SIMD, 0.25 us per 32-column step and 16 x 16 outputs (a
 // quad's 16 x 4: a quarter, times 1.24), not less than a step's loads (0.09 us and 0.034 per
 // operand piece), W's stream (6.3 TB/s) or the operands' reads from the L2 (8.7 TB/s), then the
-// reduction of the slices (1.1 us and 3.1 TB/s). Fitted to a sweep of the Qwen3-0.6B and -8B
-// projections at 4 to 2048 rows (106 shapes, 21 tiles x 11 slice counts): the picked pair takes
-// 1.03 of the best one's time on average, 1.24 at worst (4 rows); 64 x 64 tiles (quads up to 32
-// rows) in slices to 8 wavefronts per CU, the rule before, 1.58 and 3.5. 333 x 24576 x 4096:
-// 1654 -> 1080 us (1045 at the f64 rate of a large product); 20 x 1024 x 2048: 20 -> 9.3.
+// reduction of the slices (1.1 us and 3.1 TB/s); up to 16 rows, where W's stream is the bound, 1.08
+// times it where all slices start on the same memory channels (rows of whole 4 KiB, slices of whole
+// KiB: 24576 x 4096 by 5 in 8 slices 73 us, in 5 54). Against a sweep of the projections of the
+// Qwen3 shapes by 2 to 2048 rows (962 shapes, 5 tiles and the quads x 9 slice counts) the picked pair
+// takes 1.8 % longer than the best one on average and 28 % at worst (4096 x 2048 by 17), and 0.66 of
+// the rule before, 64 x 64 tiles (quads up to 32 rows) in slices to 8 wavefronts per CU (at worst 1.11,
+// 4096 x 2048 by 2 to 4). 333 x 24576 x 4096: 1654 -> 1080 us (1045 at the f64 rate of a large
+// product); 20 x 1024 x 2048: 20 -> 9.3.
 static ExactPlan exact_plan(uint64_t rows, uint64_t cols, uint64_t n, uint32_t cus, uint32_t ks, uint64_t ws_bytes) {
     ExactPlan best;
     double best_us = 1e30;
@@ -475,7 +478,10 @@ static ExactPlan exact_plan(uint64_t rows, uint64_t cols, uint64_t n, uint32_t c
             const double stream = 2.0 + 2.0 * rows * cols / 6.3e6, reads = (double)(tiles * steps) * pieces * 1024 / 8.7e6;
             double us = 2.0 + (double)((steps + slices - 1) / slices) * std::cbrt(work * work * work + loads * loads * loads);
             us = std::sqrt(std::sqrt(us * us * us * us + stream * stream * stream * stream + reads * reads * reads * reads));
-            if (slices > 1) us += 1.1 + (double)slices * n * rows * 8 / 3.1e6;
+            if (slices > 1) {
+                if (k.quads && n <= 16 && cols % 2048 == 0 && steps % slices == 0 && steps / slices % 16 == 0) us *= 1.08;
+                us += 1.1 + (double)slices * n * rows * 8 / 3.1e6;
+            }
             if (us < best_us) best_us = us, best = {&k, slices, tiles};
         }
     }
