@@ -264,7 +264,9 @@ typedef struct x0ne_greedy x0ne_greedy;
      serves a dense or MoE model decoding one sequence with 1, 2, 4 or 8 q
      heads per kv head (X0NE_ERR_NOT_IMPLEMENTED otherwise).
      X0NE_SUMS_F32 is the fp32-accumulating path (the reference engine's arithmetic: f32 sums,
-     matrix-core prefill passes).
+     matrix-core prefill passes). In a single-sequence engine the rows of a pass choose how its
+     GEMMs cut their sums, so a prompt position's bits depend on how many rows its pass has, those
+     behind it included; with max_batch > 1 they do not depend on the other sequences.
      X0NE_SUMS_DEFAULT (0, what EngineOptions { max_ctx } gives) is the exact mode wherever the
      engine can serve it, else the f32 path (max_batch > 1).
    - prefill_chunk: prompt rows per prefill pass (engine.rs:67, PREFILL_CHUNK); 0 takes

@@ -46,8 +46,15 @@ namespace {
 constexpr uint64_t PREFILL_CHUNK = 2048;
 // The exact mode's prefill GEMM: f64 parts of up to this many bytes (a short pass cuts K into
 // slices to fill the chip).
-constexpr uint32_t FEW_ROWS = 32;
 constexpr uint64_t EXACT_PARTS_BYTES = 64ull << 20;
+// Rows of a single-sequence f32 engine's pass that the few-row GEMM takes; more go through the tiled
+// one. A prompt through two layers, few-row against tiled, us: 8B 24 rows 329 / 355, 32 346 / 358,
+// 33 410 / 364, 64 456 / 380; 32B 24 593 / 588, 32 616 / 583, 33 816 / 582; 0.6B 32 188 / 197, 48
+// 214 / 205.
+constexpr uint32_t FEW_ROWS = 32;
+// The same in a batched engine. Prompts that share a pass have more rows each, so that a sequence's GEMMs
+// are the tiled ones in one piece whether it has the pass to itself or not: the same bits.
+constexpr uint32_t BATCH_FEW_ROWS = 64;
 constexpr uint64_t MAX_BATCH = 64;  // the few-row GEMM's most rows
 constexpr uint32_t ARGMAX_SLICES = 64;  // blocks per logits row of the batched step's argmax
 constexpr uint64_t MOE_MAX_EXPERTS = 1024;  // kernels/src/lib.rs:147 (moe.hip)
@@ -969,8 +976,8 @@ x0ne_status launch_rows(x0ne_engine* e, const void* fn, dim3 grid, dim3 block, v
 }
 
 // Y[n][rows] = X[n][cols] W^T on arena slices (Gpu::gemm, bf16 out). A panel prefill pass
-// (ppanel) passes W's panel copy and X in panels: up to 64 rows the few-row GEMM, more the tiled
-// GEMM. The exact mode's: the f64-sum GEMM (its K slices' parts in p_parts). Y is row-major.
+// (ppanel) passes W's panel copy and X in panels: up to FEW_ROWS rows (batched engines
+// BATCH_FEW_ROWS) the few-row GEMM, more the tiled GEMM. The exact mode's: the f64-sum GEMM (its K slices' parts in p_parts). Y is row-major.
 x0ne_status gemm(x0ne_engine* e, x0ne_slice w, x0ne_slice w_panels, uint64_t rows, uint64_t cols, x0ne_slice x,
                  uint64_t n, x0ne_slice y) {
     if (e->f64_sums)
@@ -980,7 +987,7 @@ x0ne_status gemm(x0ne_engine* e, x0ne_slice w, x0ne_slice w_panels, uint64_t row
     if (!e->ppanel)
         return gemv_rows(e->gpu, (uint64_t)(uintptr_t)e->d(w), rows, cols, (uint64_t)(uintptr_t)e->d(x), n,
                          (uint64_t)(uintptr_t)e->d(y), false, work);
-    if (n <= (e->max_batch > 1 ? 64u : FEW_ROWS)) return skinny(e->gpu, e->d(w_panels), rows, cols, e->d(x), n, e->d(y), 0, PANEL_X | PANEL_W);
+    if (n <= (e->max_batch > 1 ? BATCH_FEW_ROWS : FEW_ROWS)) return skinny(e->gpu, e->d(w_panels), rows, cols, e->d(x), n, e->d(y), 0, PANEL_X | PANEL_W);
     return tiled_gemm(e->gpu, 0, X0NE_GEMM_W_PANELS | X0NE_GEMM_X_PANELS, e->d(w_panels), rows, cols, e->d(x), n,
                       e->d(y), false, work);
 }
@@ -2148,11 +2155,10 @@ x0ne_status batch_prefill(x0ne_engine* e, const uint32_t* prompts, size_t np, ui
         X0NE_TRY(put_prompt(e, prompts + (size_t)b * np, np, b));
     // Prompts that fit a pass several at a time go together (chunk / pass_rows(np) of them), the
     // others one sequence at a time in passes of up to chunk rows. Only
-    // prompts of more than 64 rows: a sequence alone then runs the same tiled GEMM as the shared
-    // pass (64 rows or fewer take the few-row kernel), so each sequence's bits do not depend on
-    // the batch.
+    // prompts of more than BATCH_FEW_ROWS rows: a sequence alone then runs the same tiled GEMM as the
+    // shared pass, so each sequence's bits do not depend on the batch.
     const uint64_t per_pass =
-        np > 64 && np <= e->chunk ? std::max<uint64_t>(e->chunk / pass_rows(e, np), 1) : 1;
+        np > BATCH_FEW_ROWS && np <= e->chunk ? std::max<uint64_t>(e->chunk / pass_rows(e, np), 1) : 1;
     // Its logits row where the batched step leaves the others' (the last token's logits of a
     // one-token request).
     auto keep_logits = [&](uint32_t b) -> x0ne_status {

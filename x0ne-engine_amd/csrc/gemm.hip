@@ -474,6 +474,8 @@ __device__ __forceinline__ void gemm_f64(const bf16_t* __restrict__ w, const bf1
              uint32_t cols, uint32_t n, uint32_t out_f32, uint32_t ks, double* __restrict__ ws) {                 \
         gemm_f64<TF, TT>(w, x, y, rows, cols, n, out_f32, ks, ws);                                                 \
     }
+// t1 and t4 (64 x 16, 64 x 64) are for callers of the kernel table, who name them. exact_gemm does
+// without: of 962 shapes swept t4 was faster than the pick on 5, by at most 4 % (4096 x 12288 by 256).
 X0NE_GEMM_F64(x0ne_gemm_f64_t1_bf16, 4, 1)
 X0NE_GEMM_F64(x0ne_gemm_f64_t2_bf16, 4, 2)
 X0NE_GEMM_F64(x0ne_gemm_f64_t4_bf16, 4, 4)
